@@ -1224,6 +1224,42 @@ def test_paged_append_fp8(dtype, phase, T):
     assert int((vc_g.cpu() & 0x7F).eq(0x7F).sum()) > (100 if T >= 2000 else 3)
 
 
+# (cache, H, D, bs, T, phase): the one-wave kernel's shapes change at 192 and 448 pieces (16-bit: 32, 64, 128 row elements
+# per wave), at 256 and past 1024 (fp8: 32, general kernel, 64); pieces = ceil(T / 16) * ceil(H * D / 128)
+@pytest.mark.parametrize("cache,H,D,bs,T,phase", [
+    ("auto", 4, 128, 16, 752, 0), ("auto", 4, 128, 16, 753, 3), ("auto", 5, 104, 16, 700, 7), ("auto", 3, 72, 32, 1100, 1),
+    ("auto", 4, 128, 16, 1776, 5), ("auto", 4, 128, 16, 1777, 11), ("auto", 5, 104, 64, 1500, 2),
+    ("fp8", 4, 128, 16, 1, 0), ("fp8_sat", 4, 128, 16, 17, 0), ("fp8", 5, 112, 16, 800, 9), ("fp8_sat", 1, 16, 16, 400, 4),
+    ("fp8", 20, 128, 16, 192, 0), ("fp8_sat", 20, 128, 16, 193, 6), ("fp8", 20, 128, 16, 832, 15), ("fp8_sat", 20, 128, 16, 816, 2),
+    ("fp8_sat", 5, 112, 32, 3300, 13), ("fp8", 10, 208, 64, 1000, 1)])
+def test_paged_append_every_dispatched_wave_shape(cache, H, D, bs, T, phase):
+    NB = T // 6 + 60
+    dtype = torch.bfloat16 if T % 2 else torch.float16
+    say(f"paged append, dispatched shape: {cache} H={H} D={D} bs={bs} T={T} phase={phase} {dtype}")
+    g = torch.Generator().manual_seed(T + H)
+    slots = paged_slots(NB, bs, T, seed=T + 3, phase=phase, pad_frac=0.01)
+    assert len(slots) == T
+    wide = (torch.randn((T, 2 * H * D), generator=g) * 40).to(dtype)
+    key, value = (wide[:, i * H * D:(i + 1) * H * D].view(T, H, D) for i in range(2))
+    wide_g = wide.to(DEV)
+    key_g, value_g = (wide_g[:, i * H * D:(i + 1) * H * D].view(T, H, D) for i in range(2))
+    kc, vc = paged_caches_cpu(NB, H, D, bs, dtype if cache == "auto" else torch.uint8)
+    kc_g, vc_g = kc.to(DEV), vc.to(DEV)
+    if cache == "auto":
+        cache_ops.reshape_and_cache(key_g, value_g, kc_g, vc_g, slots.to(DEV))
+        orc.c_reshape_and_cache_paged(key.contiguous(), value.contiguous(), kc, vc, slots)
+    else:
+        ks, vs = torch.tensor([0.05]), torch.tensor([0.31])  # part of the quotients overflow
+        cache_ops.reshape_and_cache(key_g, value_g, kc_g, vc_g, slots.to(DEV), cache, ks.to(DEV), vs.to(DEV))
+        k8, v8 = key.contiguous(), value.contiguous()
+        if cache == "fp8_sat":  # the bytes of the saturating cast, placed by the byte-copying reference
+            k8, v8 = (torch.from_numpy(orc.c_quant_fp8_sat(x, float(sc)).reshape(T, H, D).copy()) for x, sc in ((k8, ks), (v8, vs)))
+            orc.ref_reshape_and_cache_paged(k8, v8, kc, vc, slots)
+        else:
+            orc.c_reshape_and_cache_paged(k8, v8, kc, vc, slots, float(ks), float(vs))
+    assert same_bits(kc_g, kc) and same_bits(vc_g, vc)
+
+
 def test_fp8_append_exhaustive_bf16_and_f16(golden_dir):
     """Every 16-bit input x several scales through the append kernel: 64 tokens x 1024
     elements is exactly the 65 536 bit patterns."""
