@@ -15,6 +15,8 @@ EMM_KV_ABI_VERSION = 3
 EMM_MAX_LAYERS = 96
 EMM_MAX_SEGMENTS = 128
 EMM_MAX_INLINE_IDS = 512
+EMM_MAX_INLINE_PAIRS = 480
+EMM_MAX_INLINE_PAIRS_TABLES = 112
 EMM_DTYPE_BF16 = 0
 EMM_DTYPE_F16 = 1
 EMM_FP8_SATURATE = 0x100
@@ -33,6 +35,8 @@ SIGNATURES = {
     "emm_kv_unpack_host_ids": (c_int, [_PP, c_int, c_int, c_int64, c_int64, _P, c_int64, _P, _P]),
     "emm_copy_blocks": (c_int, [_PP, c_int, c_int, c_int64, c_int64, _P, c_int64, _P]),
     "emm_kv_migrate": (c_int, [_PP, c_int64, _PP, c_int64, c_int, c_int, c_int64, _P, _P, c_int64, _P]),
+    "emm_kv_migrate_host_ids": (c_int, [_PP, c_int64, _PP, c_int64, c_int, c_int, c_int64, _P, _P, c_int64, _P]),
+    "emm_kv_unpack_dequant_fp8_host_ids": (c_int, [_PP, c_int, c_int64, c_int64, _P, c_int64, _P, _P, _P, c_int, _P]),
     "emm_kv_unpack_dequant_fp8": (c_int, [_PP, c_int, c_int64, c_int64, _P, c_int64, _P, _P, _P, c_int, _P]),
     "emm_reshape_and_cache": (c_int, [_P, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int64, c_int64, _P]),
     "emm_reshape_and_cache_layers": (c_int, [_PP, _PP, _PP, _PP, c_int, _P, c_int64, c_int64, c_int64, c_int64,

@@ -33,6 +33,67 @@
 #include "emm_append_paged.inc"
 #include "emm_concat.inc"
 
+namespace {
+int unpack_dequant(void *const *layer_ptrs, int num_layers, int64_t num_blocks,
+                              int64_t chunk_elems, const int64_t *block_idx, const int64_t *host_idx, int64_t n,
+                              const void *packed_fp8, const float *k_scales,
+                              const float *v_scales, int out_dtype, emm_stream_t stream, const char *what) {
+  int rc = check_pool_args(what, (const void *const *)layer_ptrs, num_layers, 2, num_blocks,
+                           chunk_elems, n);
+  if (rc != EMM_OK) return rc;
+  if (out_dtype != EMM_DTYPE_BF16 && out_dtype != EMM_DTYPE_F16)
+    return fail(EMM_EINVAL, "%s: unknown out_dtype %d", what, out_dtype);
+  if (n == 0 || num_layers == 0 || chunk_elems == 0) return EMM_OK;
+  if ((!block_idx && !host_idx) || !packed_fp8 || !k_scales || !v_scales)
+    return fail(EMM_EINVAL, "%s: null pointer argument", what);
+  if (chunk_elems % 16 != 0 || !aligned(packed_fp8, 16))
+    return fail(EMM_EINVAL, "%s: chunk_elems (%lld) and packed_fp8 must be multiples of 16",
+                what, (long long)chunk_elems);
+  if (chunk_elems > 0x3fffffffLL || num_blocks > 0x7fffffffLL)
+    return fail(EMM_EINVAL, "%s: chunk_elems / num_blocks too large", what);
+  LayerTable t;
+  for (int l = 0; l < num_layers; ++l) {
+    if (!aligned(layer_ptrs[l], 16))
+      return fail(EMM_EINVAL, "%s: layer_ptrs[%d] not 16-byte aligned", what, l);
+    t.base[l] = (char *)layer_ptrs[l];
+  }
+  const int64_t tile = (int64_t)kThreads * 16;
+  const int64_t tpc = (chunk_elems + tile - 1) / tile;
+  hipStream_t s = as_stream(stream);
+  const int64_t step = host_idx ? EMM_MAX_INLINE_IDS : kMaxGridY;
+  for (int64_t j0 = 0; j0 < n; j0 += step) {
+    const int64_t ny = (n - j0 < step) ? (n - j0) : step;
+    const char *packed = (const char *)packed_fp8 + j0 * chunk_elems;
+    const int64_t *idx = block_idx ? block_idx + j0 : nullptr;
+    const int64_t stride = n * chunk_elems;
+    const bool grouped = ny >= 1024 && ((2 * num_layers) << 8) <= kMaxGridY; // groups of 256 blocks, as in unpack
+    const uint32_t remap = xcd_mapping(kMapDequant, ny, tpc, num_blocks, 2 * chunk_elems);
+    const dim3 grid = grouped ? dim3((uint32_t)tpc, (uint32_t)((2 * num_layers) << 8), (uint32_t)((ny + 255) >> 8))
+                              : dim3((uint32_t)tpc, (uint32_t)ny, (uint32_t)(2 * num_layers));
+#define EMM_DQ_LAUNCH(DT, G, IN, IDS) \
+  emm_unpack_dequant_fp8_kernel<DT, G, IN><<<grid, kThreads, 0, s>>>(packed, idx, k_scales, v_scales, stride, \
+      (uint32_t)chunk_elems, (uint32_t)num_blocks, (uint32_t)ny, 8u | remap, t, IDS)
+    if (host_idx) { // at most EMM_MAX_INLINE_IDS blocks: never grouped
+      InlineIds ids;
+      for (int64_t j = 0; j < ny; ++j)
+        ids.id[j] = host_idx[j0 + j] >= 0 && host_idx[j0 + j] < num_blocks ? (uint32_t)host_idx[j0 + j] : 0xffffffffu;
+      if (out_dtype == EMM_DTYPE_BF16) EMM_DQ_LAUNCH(EMM_DTYPE_BF16, false, true, ids);
+      else EMM_DQ_LAUNCH(EMM_DTYPE_F16, false, true, ids);
+    } else if (out_dtype == EMM_DTYPE_BF16) {
+      if (grouped) EMM_DQ_LAUNCH(EMM_DTYPE_BF16, true, false, NoIds{});
+      else EMM_DQ_LAUNCH(EMM_DTYPE_BF16, false, false, NoIds{});
+    } else {
+      if (grouped) EMM_DQ_LAUNCH(EMM_DTYPE_F16, true, false, NoIds{});
+      else EMM_DQ_LAUNCH(EMM_DTYPE_F16, false, false, NoIds{});
+    }
+#undef EMM_DQ_LAUNCH
+    const int rc2 = check_launch(what);
+    if (rc2 != EMM_OK) return rc2;
+  }
+  return EMM_OK;
+}
+} // namespace
+
 // ============================================================================
 // C ABI
 // ============================================================================
@@ -145,48 +206,31 @@ int emm_kv_unpack_dequant_fp8(void *const *layer_ptrs, int num_layers, int64_t n
                               int64_t chunk_elems, const int64_t *block_idx, int64_t n,
                               const void *packed_fp8, const float *k_scales,
                               const float *v_scales, int out_dtype, emm_stream_t stream) {
-  const char *what = "emm_kv_unpack_dequant_fp8";
-  int rc = check_pool_args(what, (const void *const *)layer_ptrs, num_layers, 2, num_blocks,
-                           chunk_elems, n);
+  return unpack_dequant(layer_ptrs, num_layers, num_blocks, chunk_elems, block_idx, nullptr, n, packed_fp8, k_scales,
+                        v_scales, out_dtype, stream, "emm_kv_unpack_dequant_fp8");
+}
+
+int emm_kv_unpack_dequant_fp8_host_ids(void *const *layer_ptrs, int num_layers, int64_t num_blocks,
+                                       int64_t chunk_elems, const int64_t *host_block_idx, int64_t n,
+                                       const void *packed_fp8, const float *k_scales,
+                                       const float *v_scales, int out_dtype, emm_stream_t stream) {
+  return unpack_dequant(layer_ptrs, num_layers, num_blocks, chunk_elems, nullptr, host_block_idx, n, packed_fp8, k_scales,
+                        v_scales, out_dtype, stream, "emm_kv_unpack_dequant_fp8_host_ids");
+}
+
+int emm_kv_migrate_host_ids(const void *const *src_layer_ptrs, int64_t src_num_blocks,
+                            void *const *dst_layer_ptrs, int64_t dst_num_blocks, int num_layers,
+                            int num_kv, int64_t chunk_bytes, const int64_t *host_src_idx,
+                            const int64_t *host_dst_idx, int64_t n, emm_stream_t stream) {
+  const char *what = "emm_kv_migrate_host_ids";
+  int rc = check_pool_args(what, src_layer_ptrs, num_layers, num_kv, src_num_blocks, chunk_bytes, n);
   if (rc != EMM_OK) return rc;
-  if (out_dtype != EMM_DTYPE_BF16 && out_dtype != EMM_DTYPE_F16)
-    return fail(EMM_EINVAL, "%s: unknown out_dtype %d", what, out_dtype);
-  if (n == 0 || num_layers == 0 || chunk_elems == 0) return EMM_OK;
-  if (!block_idx || !packed_fp8 || !k_scales || !v_scales)
-    return fail(EMM_EINVAL, "%s: null pointer argument", what);
-  if (chunk_elems % 16 != 0 || !aligned(packed_fp8, 16))
-    return fail(EMM_EINVAL, "%s: chunk_elems (%lld) and packed_fp8 must be multiples of 16",
-                what, (long long)chunk_elems);
-  if (chunk_elems > 0x3fffffffLL || num_blocks > 0x7fffffffLL)
-    return fail(EMM_EINVAL, "%s: chunk_elems / num_blocks too large", what);
-  LayerTable t;
-  for (int l = 0; l < num_layers; ++l) {
-    if (!aligned(layer_ptrs[l], 16))
-      return fail(EMM_EINVAL, "%s: layer_ptrs[%d] not 16-byte aligned", what, l);
-    t.base[l] = (char *)layer_ptrs[l];
-  }
-  const int64_t tile = (int64_t)kThreads * 16;
-  const int64_t tpc = (chunk_elems + tile - 1) / tile;
-  hipStream_t s = as_stream(stream);
-  for (int64_t j0 = 0; j0 < n; j0 += kMaxGridY) {
-    const int64_t ny = (n - j0 < kMaxGridY) ? (n - j0) : kMaxGridY;
-    const char *packed = (const char *)packed_fp8 + j0 * chunk_elems;
-    const int64_t *idx = block_idx + j0;
-    const int64_t stride = n * chunk_elems;
-    const bool grouped = ny >= 1024 && ((2 * num_layers) << 8) <= kMaxGridY; // groups of 256 blocks, as in unpack
-    const uint32_t remap = xcd_mapping(kMapDequant, ny, tpc, num_blocks, 2 * chunk_elems);
-    const dim3 grid = grouped ? dim3((uint32_t)tpc, (uint32_t)((2 * num_layers) << 8), (uint32_t)((ny + 255) >> 8))
-                              : dim3((uint32_t)tpc, (uint32_t)ny, (uint32_t)(2 * num_layers));
-#define EMM_DQ_LAUNCH(DT, G) \
-  emm_unpack_dequant_fp8_kernel<DT, G><<<grid, kThreads, 0, s>>>(packed, idx, k_scales, v_scales, stride, \
-      (uint32_t)chunk_elems, (uint32_t)num_blocks, (uint32_t)ny, 8u | remap, t)
-    if (out_dtype == EMM_DTYPE_BF16) { if (grouped) EMM_DQ_LAUNCH(EMM_DTYPE_BF16, true); else EMM_DQ_LAUNCH(EMM_DTYPE_BF16, false); }
-    else { if (grouped) EMM_DQ_LAUNCH(EMM_DTYPE_F16, true); else EMM_DQ_LAUNCH(EMM_DTYPE_F16, false); }
-#undef EMM_DQ_LAUNCH
-    const int rc2 = check_launch(what);
-    if (rc2 != EMM_OK) return rc2;
-  }
-  return EMM_OK;
+  rc = check_pool_args(what, (const void *const *)dst_layer_ptrs, num_layers, num_kv, dst_num_blocks, chunk_bytes, n);
+  if (rc != EMM_OK) return rc;
+  if (n == 0 || num_layers == 0 || num_kv == 0 || chunk_bytes == 0) return EMM_OK;
+  if (!host_src_idx || !host_dst_idx) return fail(EMM_EINVAL, "%s: null index array", what);
+  return migrate_host(src_layer_ptrs, src_num_blocks, dst_layer_ptrs, dst_num_blocks, num_layers, num_kv, chunk_bytes,
+                      host_src_idx, host_dst_idx, n, as_stream(stream), what);
 }
 
 int emm_reshape_and_cache(const void *key, const void *value, void *key_cache,

@@ -12,7 +12,8 @@ import numpy as np
 import torch
 
 from . import _lib
-from ._lib import (EMM_DTYPE_BF16, EMM_DTYPE_F16, EMM_FP8_SATURATE, EMM_MAX_INLINE_IDS, EMM_MAX_LAYERS,
+from ._lib import (EMM_DTYPE_BF16, EMM_DTYPE_F16, EMM_FP8_SATURATE, EMM_MAX_INLINE_IDS, EMM_MAX_INLINE_PAIRS,
+                   EMM_MAX_INLINE_PAIRS_TABLES, EMM_MAX_LAYERS,
                    EMM_MAX_SEGMENTS, check,
                    ptr_table)
 
@@ -140,6 +141,8 @@ class PoolView:
         self.chunk_elems = int(np.prod(self.block_shape, dtype=np.int64)) if self.block_shape else 1
         self.chunk_bytes = self.chunk_elems * self.elem_bytes
         self.ptrs = [t.data_ptr() for t in layers]
+        step = self.num_kv * self.num_blocks * self.chunk_bytes
+        self.equal_planes = all(p == self.ptrs[0] + l * step for l, p in enumerate(self.ptrs))
         # the host pointer tables the entry points take, built once (the layers stay where they are)
         self._groups = [(l0, ptr_table(self.ptrs[l0:l0 + EMM_MAX_LAYERS]))
                         for l0 in range(0, len(layers), EMM_MAX_LAYERS)]
@@ -262,8 +265,21 @@ def kv_migrate(src: PoolView, src_indices: IndexLike, dst: PoolView, dst_indices
         raise ValueError("kv_migrate: pools differ in layers / kv / chunk size / device")
     if src.on_host and dst.on_host:
         raise ValueError("kv_migrate: at least one pool must live in GPU memory")
-    si = block_index_tensor(src_indices, src.num_blocks, src.device)
-    di = block_index_tensor(dst_indices, dst.num_blocks, dst.device)
+    hs = host_block_ids(src_indices, src.num_blocks)
+    hd = host_block_ids(dst_indices, dst.num_blocks)
+    if hs is not None and hd is not None and not (src.on_host or dst.on_host):
+        # two host tables: the ids travel in the argument block while that takes at most two launches
+        if hs.size != hd.size:
+            raise ValueError(f"Block count mismatch: src={hs.size}, dst={hd.size}")
+        per_launch = EMM_MAX_INLINE_PAIRS if src.equal_planes and dst.equal_planes else EMM_MAX_INLINE_PAIRS_TABLES
+        if hs.size <= 2 * per_launch:
+            stream = _stream_ptr(src.device)
+            for (l0, st), (_, dt) in zip(src.layer_groups(), dst.layer_groups()):
+                check(lib.emm_kv_migrate_host_ids(st, src.num_blocks, dt, dst.num_blocks, len(st), src.num_kv, src.chunk_bytes,
+                                                  hs.ctypes.data, hd.ctypes.data, hs.size, stream), "emm_kv_migrate_host_ids")
+            return
+    si = block_index_tensor(hs if hs is not None else src_indices, src.num_blocks, src.device)
+    di = block_index_tensor(hd if hd is not None else dst_indices, dst.num_blocks, dst.device)
     if si.numel() != di.numel():
         raise ValueError(f"Block count mismatch: src={si.numel()}, dst={di.numel()}")
     stream = _stream_ptr(src.device)
@@ -324,8 +340,12 @@ def kv_unpack_dequant_fp8(pool: PoolView, block_indices: IndexLike, packed_fp8: 
     if packed_fp8.element_size() != 1:
         raise TypeError("packed_fp8 must be a 1-byte tensor (float8_e4m3fn or uint8)")
     code = _half_code(pool.dtype, "kv_unpack_dequant_fp8")
-    idx = block_index_tensor(block_indices, pool.num_blocks, pool.device)
-    n = idx.numel()
+    host = host_block_ids(block_indices, pool.num_blocks)
+    if host is not None and host.size <= 2 * EMM_MAX_INLINE_IDS and not pool.on_host:  # ids in the argument block
+        n, table_arg, fn, what = host.size, host.ctypes.data, lib.emm_kv_unpack_dequant_fp8_host_ids, "emm_kv_unpack_dequant_fp8_host_ids"
+    else:
+        idx = block_index_tensor(host if host is not None else block_indices, pool.num_blocks, pool.device)
+        n, table_arg, fn, what = idx.numel(), idx.data_ptr(), lib.emm_kv_unpack_dequant_fp8, "emm_kv_unpack_dequant_fp8"
     if packed_fp8.numel() != pool.num_layers * 2 * n * pool.chunk_elems:
         raise ValueError("kv_unpack_dequant_fp8: packed buffer size does not match the pool geometry")
     packed_fp8 = packed_fp8.contiguous()
@@ -334,9 +354,8 @@ def kv_unpack_dequant_fp8(pool: PoolView, block_indices: IndexLike, packed_fp8: 
     stream = _stream_ptr(pool.device)
     plane = 2 * n * pool.chunk_elems
     for l0, table in pool.layer_groups():
-        check(lib.emm_kv_unpack_dequant_fp8(table, len(table), pool.num_blocks, pool.chunk_elems, idx.data_ptr(), n,
-                                            packed_fp8.data_ptr() + l0 * plane, ks.data_ptr() + 4 * l0,
-                                            vs.data_ptr() + 4 * l0, code, stream), "emm_kv_unpack_dequant_fp8")
+        check(fn(table, len(table), pool.num_blocks, pool.chunk_elems, table_arg, n, packed_fp8.data_ptr() + l0 * plane,
+                 ks.data_ptr() + 4 * l0, vs.data_ptr() + 4 * l0, code, stream), what)
 
 
 def _row_geometry(x: torch.Tensor, what: str):

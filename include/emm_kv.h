@@ -43,6 +43,8 @@ extern "C" {
 #define EMM_MAX_LAYERS 96   /* layer pointers carried in one kernel argument block */
 #define EMM_MAX_SEGMENTS 128 /* ragged segments carried by one emm_concat_rows launch */
 #define EMM_MAX_INLINE_IDS 512 /* block ids carried by one launch of emm_kv_*_host_ids (longer tables: several launches) */
+#define EMM_MAX_INLINE_PAIRS 480 /* (source, destination) ids carried by one launch of emm_kv_migrate_host_ids */
+#define EMM_MAX_INLINE_PAIRS_TABLES 112 /* the same for pools whose planes are not equally spaced */
 
 /* error codes */
 #define EMM_OK 0
@@ -138,6 +140,16 @@ int emm_kv_migrate(const void *const *src_layer_ptrs, int64_t src_num_blocks,
                    int num_layers, int num_kv, int64_t chunk_bytes,
                    const int64_t *src_idx, const int64_t *dst_idx, int64_t n,
                    emm_stream_t stream);
+/* The same with both block tables given as HOST arrays of n ids: the ids travel in the kernel argument block, so no
+ * device-side table and no host-to-device copy is needed (EMM_MAX_INLINE_PAIRS pairs per launch if the planes of
+ * each pool are equally spaced, EMM_MAX_INLINE_PAIRS_TABLES otherwise; a longer table takes several launches).
+ * A pair with an id out of range is skipped. A launch recorded into a HIP graph keeps the ids it was recorded with. */
+int emm_kv_migrate_host_ids(const void *const *src_layer_ptrs, int64_t src_num_blocks,
+                            void *const *dst_layer_ptrs, int64_t dst_num_blocks,
+                            int num_layers, int num_kv, int64_t chunk_bytes,
+                            const int64_t *host_src_idx, const int64_t *host_dst_idx,
+                            int64_t n, emm_stream_t stream);
+
 
 /*
  * dequant-unpack — scatter an fp8-e4m3fn transfer buffer
@@ -154,6 +166,15 @@ int emm_kv_unpack_dequant_fp8(void *const *layer_ptrs, int num_layers,
                               const void *packed_fp8, const float *k_scales,
                               const float *v_scales, int out_dtype,
                               emm_stream_t stream);
+/* The same with the block table given as a HOST array: the ids travel in the kernel argument block, as in
+ * emm_kv_unpack_host_ids (EMM_MAX_INLINE_IDS ids per launch). */
+int emm_kv_unpack_dequant_fp8_host_ids(void *const *layer_ptrs, int num_layers,
+                                       int64_t num_blocks, int64_t chunk_elems,
+                                       const int64_t *host_block_idx, int64_t n,
+                                       const void *packed_fp8, const float *k_scales,
+                                       const float *v_scales, int out_dtype,
+                                       emm_stream_t stream);
+
 
 /*
  * reshape_and_cache (flash layout) — append: for token t with

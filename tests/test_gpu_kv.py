@@ -435,6 +435,50 @@ def test_cache_ops_swap_blocks_between_gpu_and_pinned_host():
         cache_ops.swap_blocks(cpu, cpu, out_pairs)
 
 
+@pytest.mark.parametrize("equal", [True, False], ids=["equally spaced planes", "separate layers"])
+@pytest.mark.parametrize("bs,H,D,n", [(16, 4, 128, 1), (16, 4, 128, 17), (16, 2, 64, 112), (16, 2, 64, 113), (16, 4, 128, 225),
+                                      (16, 2, 64, 480), (16, 2, 64, 481), (8, 1, 40, 960), (8, 1, 40, 961), (3, 1, 7, 130),
+                                      (16, 8, 256, 100)])
+def test_migrate_with_host_tables(equal, bs, H, D, n):
+    """Both tables as lists: the ids travel in the argument block, in one launch, in two, or (past two launches) through
+    device tables; against torch's indexing on the host."""
+    L, NBs, NBd = 3, 1100, 1030
+    say(f"migrate, host tables: equal={equal} bs={bs} H={H} D={D} n={n}")
+    src_c, dst_c = cpu_pool(L, NBs, bs, H, D, torch.bfloat16, n), cpu_pool(L, NBd, bs, H, D, torch.bfloat16, 0, fill=-1.0)
+    src, dst = to_dev(src_c, equal), to_dev(dst_c, equal)
+    pools = PoolView(src), PoolView(dst)
+    if equal:
+        assert pools[0].equal_planes and pools[1].equal_planes
+    g = torch.Generator().manual_seed(n)
+    si = torch.randperm(NBs, generator=g)[:n].tolist()
+    di = torch.randperm(NBd, generator=g)[:n].tolist()
+    si[0] -= NBs  # counted from the end
+    kv_ops.kv_migrate(pools[0], si, pools[1], di)
+    for l in range(L):
+        dst_c[l][:, di] = src_c[l][:, si]
+        assert same_bits(dst[l], dst_c[l]) and same_bits(src[l], src_c[l]), f"layer {l}"
+    with pytest.raises(IndexError):
+        kv_ops.kv_migrate(pools[0], [NBs], pools[1], [0])
+    with pytest.raises(ValueError):
+        kv_ops.kv_migrate(pools[0], si, pools[1], di[:-1])
+
+
+@pytest.mark.parametrize("n", [1, 96, 512, 513, 1024, 1025])
+def test_dequant_unpack_with_host_table(n):
+    """A list travels in the argument block (1, 2 launches) or, past that, through a device table: the same result as
+    with the table on the device."""
+    L, NB, bs, H, D = 2, 1100, 16, 1, 64
+    g = torch.Generator().manual_seed(n)
+    packed = torch.randint(0, 256, (L, 2, n, bs, H, D), dtype=torch.uint8, generator=g).to(DEV)
+    ids = torch.randperm(NB, generator=g)[:n]
+    ks, vs = torch.tensor([0.02, 0.3], device=DEV), torch.tensor([0.5, 0.07], device=DEV)
+    got, want = (to_dev(cpu_pool(L, NB, bs, H, D, torch.bfloat16, 0, fill=-1.0)) for _ in range(2))
+    kv_ops.kv_unpack_dequant_fp8(PoolView(got), ids.tolist(), packed, ks, vs)
+    kv_ops.kv_unpack_dequant_fp8(PoolView(want), ids.to(DEV), packed, ks, vs)
+    for l in range(L):
+        assert same_bits(got[l], want[l].cpu()), f"n={n} layer {l}"
+
+
 def test_migrate_equals_pack_then_unpack():
     L, NBs, NBd = 4, 40, 24
     src_c = cpu_pool(L, NBs, 16, 4, 128, torch.bfloat16, 10)
