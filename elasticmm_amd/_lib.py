@@ -6,10 +6,11 @@ the caller gets an exception.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 from ctypes import c_char_p, c_float, c_int, c_int64, c_void_p, POINTER
 
-from .build import hooks_library_path, library_path
+from .build import frontend_path, hooks_library_path, library_path
 
 EMM_KV_ABI_VERSION = 3
 EMM_MAX_LAYERS = 96
@@ -79,6 +80,27 @@ class EmmError(RuntimeError):
     """An entry point of libemm_kv.so returned a non-zero code."""
 
 
+_frontend_module = None
+
+
+def _bind_frontend(lib: ctypes.CDLL) -> None:
+    """``lib.frontend``: the native host side of the per-layer appends (csrc/emm_frontend.cpp) over this library's
+    entry points."""
+    global _frontend_module
+    if _frontend_module is None:
+        path = frontend_path()
+        if not os.path.exists(path):
+            raise RuntimeError(f"{path} is missing: the native host side has not been built "
+                               "(run `python -m elasticmm_amd.build`)")
+        spec = importlib.util.spec_from_file_location("_emm_frontend", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _frontend_module = module
+    address = lambda fn: ctypes.cast(fn, c_void_p).value  # noqa: E731
+    lib.frontend = _frontend_module.Frontend(address(lib.emm_reshape_and_cache), address(lib.emm_reshape_and_cache_fp8),
+                                             address(lib.emm_reshape_and_cache_paged))
+
+
 def load() -> ctypes.CDLL:
     """Load libemm_kv.so once; raises if it has not been built."""
     global _lib
@@ -91,10 +113,7 @@ def load() -> ctypes.CDLL:
             "(run `python -m elasticmm_amd.build`). There is no CPU fallback.")
     # torch carries its own copy of the HIP runtime and exports its symbols globally. Streams and device pointers
     # come from torch, so the library has to bind to that copy: torch is loaded before the library is.
-    try:
-        import torch  # noqa: F401
-    except ImportError:
-        pass
+    import torch  # noqa: F401
     lib = ctypes.CDLL(path)
     for name, (res, args) in SIGNATURES.items():
         fn = getattr(lib, name)  # AttributeError if the symbol is not exported
@@ -103,6 +122,7 @@ def load() -> ctypes.CDLL:
     ver = lib.emm_abi_version()
     if ver != EMM_KV_ABI_VERSION:
         raise RuntimeError(f"libemm_kv.so ABI version {ver}, expected {EMM_KV_ABI_VERSION}")
+    _bind_frontend(lib)
     _lib = lib
     return lib
 
@@ -115,15 +135,13 @@ def load_hooks() -> ctypes.CDLL:
     path = hooks_library_path()
     if not os.path.exists(path):
         raise RuntimeError(f"{path} is missing (run `python -m elasticmm_amd.build`)")
-    try:
-        import torch  # noqa: F401
-    except ImportError:
-        pass
+    import torch  # noqa: F401
     lib = ctypes.CDLL(path)
     for name, (res, args) in {**SIGNATURES, **HOOK_SIGNATURES}.items():
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
+    _bind_frontend(lib)
     _hooks = lib
     return lib
 

@@ -13,7 +13,7 @@ from typing import List, Optional, Sequence
 import numpy as np
 import torch
 
-from . import kv_ops
+from . import _lib, kv_ops
 from .kv_ops import PoolView
 
 # kv_cache_dtype strings of the fp8 KV cache. "fp8" / "fp8_e4m3" is the cast torch performs,
@@ -22,6 +22,10 @@ from .kv_ops import PoolView
 # kernels (the variants the reference leaves open at elasticmm/engine/v0/worker.py:194); it has to be
 # asked for by name.
 _FP8_MODES = {"fp8": False, "fp8_e4m3": False, "fp8_sat": True, "fp8_e4m3_sat": True}
+
+
+# the same names as the native host side takes them (0: copy, 1: torch's cast, 2: saturating)
+_NATIVE_MODES = {"auto": 0, **{name: 2 if sat else 1 for name, sat in _FP8_MODES.items()}}
 
 
 def reshape_and_cache_flash(key: torch.Tensor, value: torch.Tensor, key_cache: torch.Tensor,
@@ -34,6 +38,13 @@ def reshape_and_cache_flash(key: torch.Tensor, value: torch.Tensor, key_cache: t
     dtype == key dtype, bit copy), "fp8" / "fp8_e4m3" (cache is 1 byte wide and
     is written as ``e4m3fn(float(x) / scale)``, torch's cast) or "fp8_sat" / "fp8_e4m3_sat" (the
     same with the quotient clamped to [-448, 448] first)."""
+    mode = _NATIVE_MODES.get(kv_cache_dtype)
+    if mode is not None:  # the usual forms are checked and launched in native code; 0: not one of them
+        rc = _lib.load().frontend.append_flash(key, value, key_cache, value_cache, slot_mapping, mode, k_scale, v_scale)
+        if rc:
+            if rc < 0:
+                _lib.check(rc, "reshape_and_cache_flash")
+            return
     if kv_cache_dtype == "auto":
         if key_cache.element_size() != key.element_size():
             raise ValueError("kv_cache_dtype='auto' needs a cache of the key's element size")
@@ -60,6 +71,13 @@ def reshape_and_cache(key: torch.Tensor, value: torch.Tensor, key_cache: torch.T
     """The append of vLLM's PagedAttention backends (its default attention path on ROCm): key, value
     ``[num_tokens, num_heads, head_size]``; key_cache ``[num_blocks, num_heads, head_size // x, block_size, x]``,
     value_cache ``[num_blocks, num_heads, head_size, block_size]``, x = 16 // cache element size."""
+    mode = _NATIVE_MODES.get(kv_cache_dtype)
+    if mode is not None:
+        rc = _lib.load().frontend.append_paged(key, value, key_cache, value_cache, slot_mapping, mode, k_scale, v_scale)
+        if rc:
+            if rc < 0:
+                _lib.check(rc, "reshape_and_cache")
+            return
     if kv_cache_dtype == "auto":
         if key_cache.element_size() != key.element_size():
             raise ValueError("kv_cache_dtype='auto' needs a cache of the key's element size")

@@ -1304,6 +1304,56 @@ def test_paged_append_every_dispatched_wave_shape(cache, H, D, bs, T, phase):
     assert same_bits(kc_g, kc) and same_bits(vc_g, vc)
 
 
+@pytest.mark.parametrize("layout", ["flash", "paged"])
+@pytest.mark.parametrize("cache", ["auto", "fp8", "fp8_sat"])
+def test_native_append_takes_the_usual_calls_only(layout, cache):
+    """The native host side launches the usual calls; anything else is left, untouched, to the Python operators, which
+    give the same bytes or the error they always gave."""
+    T, H, D, NB, bs = 9, 2, 64, 5, 16
+    g = torch.Generator().manual_seed(5)
+    key, value = (torch.randn((T, H, D), generator=g).to(torch.bfloat16).to(DEV) for _ in range(2))
+    slots = torch.randperm(NB * bs, generator=g)[:T].to(DEV)
+    dt = torch.bfloat16 if cache == "auto" else torch.uint8
+    x = 16 // torch.empty((), dtype=dt).element_size()
+    shapes = [(NB, bs, H, D)] * 2 if layout == "flash" else [(NB, H, D // x, bs, x), (NB, H, D, bs)]
+    caches = lambda: [torch.full(sh, 7, dtype=dt, device=DEV) for sh in shapes]  # noqa: E731
+    one = torch.tensor([0.05], device=DEV)
+    native = getattr(_lib.load().frontend, "append_" + layout)
+    op = cache_ops.reshape_and_cache_flash if layout == "flash" else cache_ops.reshape_and_cache
+    mode = cache_ops._NATIVE_MODES[cache]
+    wide = torch.zeros((T, 3 * H * D), dtype=torch.bfloat16, device=DEV)
+    wide[:, H * D:2 * H * D] = key.view(T, -1)
+    strided = wide[:, H * D:2 * H * D].view(T, H, D)
+    want = caches()
+    op(key, value, *want, slots, cache, one, one)
+    for k in (key, strided):
+        c = caches()
+        assert native(k, value, *c, slots, mode, one, one) == 1
+        assert same_bits(c[0], want[0]) and same_bits(c[1], want[1])
+
+    class Sub(torch.Tensor):
+        pass
+
+    odd = [(key.as_subclass(Sub), value, slots, one), (key, value, slots.repeat_interleave(2)[::2], one),
+           (key.permute(2, 1, 0).contiguous().permute(2, 1, 0), value, slots, one), (key, value, slots.int(), one),
+           (key, value, slots[:-1], one), (key[:0], value[:0], slots, one), (key, value[:, :1], slots, one),
+           (key, value, slots.cpu(), one)]
+    if layout == "flash":
+        odd.append((key.view(T, H * D), value.view(T, H * D), slots, one))
+    if cache != "auto":
+        odd += [(key, value, slots, one.double()), (key, value, slots, None), (key, value, slots, 0.05), (key.float(), value.float(), slots, one)]
+    for n, (k, v, s, sc) in enumerate(odd):
+        c = caches()
+        assert native(k, v, *c, s, mode, sc, sc) == 0, f"odd call {n}"
+        assert all(bool((t == 7).all()) for t in c), f"odd call {n} wrote"
+        try:
+            op(k, v, *c, s, cache, sc, sc)
+        except (ValueError, TypeError, RuntimeError):
+            continue
+        if k.numel():
+            assert same_bits(c[0], want[0]) and same_bits(c[1], want[1]), f"odd call {n}"
+
+
 def test_fp8_append_exhaustive_bf16_and_f16(golden_dir):
     """Every 16-bit input x several scales through the append kernel: 64 tokens x 1024
     elements is exactly the 65 536 bit patterns."""
