@@ -18,6 +18,7 @@ EMM_MAX_SEGMENTS = 128
 EMM_MAX_INLINE_IDS = 512
 EMM_MAX_INLINE_PAIRS = 480
 EMM_MAX_INLINE_PAIRS_TABLES = 112
+EMM_MAX_SLOT_WORDS = 960
 EMM_DTYPE_BF16 = 0
 EMM_DTYPE_F16 = 1
 EMM_FP8_SATURATE = 0x100
@@ -54,6 +55,7 @@ SIGNATURES = {
                                             c_int64, c_int, c_int, _P, _P, _P]),
     "emm_reshape_and_cache_paged_layers": (c_int, [_PP, _PP, _PP, _PP, c_int, _P, c_int64, c_int, c_int, c_int,
                                                    c_int64, c_int64, c_int64, c_int, c_int, _P, _P, _P]),
+    "emm_slot_mapping": (c_int, [_P, _P, _P, c_int, _P, c_int64, c_int, c_int64, _P, _P]),
     "emm_concat_rows": (c_int, [_PP, _I64P, c_int, _P, c_int64, _P]),
     "emm_stream_copy": (c_int, [_P, _P, c_int64, _P]),
 }

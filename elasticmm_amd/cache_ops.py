@@ -8,6 +8,7 @@ order so an attention backend can call them unchanged.
 """
 from __future__ import annotations
 
+from array import array
 from typing import List, Optional, Sequence
 
 import numpy as np
@@ -183,6 +184,50 @@ def swap_blocks(src_kv_cache: torch.Tensor, dst_kv_cache: torch.Tensor, src_to_d
     kv_ops.kv_migrate(src, pairs[:, 0].contiguous(), dst, pairs[:, 1].contiguous())
 
 
+_MAX_SLOT_LAUNCHES = 4
+
+
+def _slot_mapping_on_device(block_tables, context_lens, query_lens, block_size, size, device) -> Optional[torch.Tensor]:
+    """The slots written by a kernel from tables in its argument block; None for whatever does not fit
+    ``_MAX_SLOT_LAUNCHES`` launches or is not a list of plain non-negative ids (the general path takes it)."""
+    launches = []
+    starts, offsets, firsts, blocks = [0], [], [], []
+    pos = 0
+    for table, ctx, q in zip(block_tables, context_lens, query_lens):
+        if type(table) is not list or type(ctx) is not int or type(q) is not int or ctx < 0 or q < 0:
+            return None
+        if q == 0:
+            continue
+        lo, hi = ctx // block_size, (ctx + q - 1) // block_size + 1
+        if hi > len(table):
+            return None
+        if 3 * len(starts) + 1 + len(blocks) + hi - lo > _lib.EMM_MAX_SLOT_WORDS:
+            if 4 + hi - lo > _lib.EMM_MAX_SLOT_WORDS or len(launches) + 2 > _MAX_SLOT_LAUNCHES:
+                return None
+            launches.append((starts, offsets, firsts, blocks))
+            starts, offsets, firsts, blocks = [pos], [], [], []
+        offsets.append(ctx - lo * block_size)
+        firsts.append(len(blocks))
+        blocks += table[lo:hi] if hi - lo > 1 else (table[lo],)
+        pos += q
+        starts.append(pos)
+    launches.append((starts, offsets, firsts, blocks))
+    try:
+        packed = [[array("q", x) for x in launch] for launch in launches]
+    except (TypeError, OverflowError):
+        return None
+    for launch in packed:
+        ids = launch[3]
+        if ids and (min(ids) < 0 or max(ids) > 0x7fffffff):
+            return None
+    out = torch.empty(size, dtype=torch.long, device=device)
+    lib, stream, ptr = _lib.load(), kv_ops._stream_ptr(out.device), out.data_ptr()
+    for n, (s, o, f, b) in enumerate(packed):
+        _lib.check(lib.emm_slot_mapping(s.buffer_info()[0], o.buffer_info()[0], f.buffer_info()[0], len(o), b.buffer_info()[0],
+                                        len(b), block_size, size if n == len(packed) - 1 else s[-1], ptr, stream), "emm_slot_mapping")
+    return out
+
+
 def compute_slot_mapping(block_tables: Sequence[Sequence[int]], context_lens: Sequence[int],
                          query_lens: Sequence[int], block_size: int, pad_to: Optional[int] = None,
                          device: Optional[torch.device] = None) -> torch.Tensor:
@@ -191,8 +236,9 @@ def compute_slot_mapping(block_tables: Sequence[Sequence[int]], context_lens: Se
     i contributes ``query_lens[i]`` tokens at positions ``context_lens[i] + k``, token at position p lives in slot
     ``block_tables[i][p // block_size] * block_size + p % block_size``. Tokens of one sequence are consecutive, so
     a prompt yields runs of consecutive slots. The result is int64, padded with -1 up to ``pad_to`` (the padded
-    entries are skipped by the append kernels), pinned when a GPU ``device`` is given and copied there without
-    blocking."""
+    entries are skipped by the append kernels). For a GPU ``device`` the slots are written there by a kernel that
+    carries the tables in its argument block; tables that do not fit are expanded in pinned memory and copied there
+    without blocking."""
     if not (len(block_tables) == len(context_lens) == len(query_lens)):
         raise ValueError("block_tables, context_lens and query_lens differ in length")
     total = int(sum(query_lens))
@@ -200,6 +246,10 @@ def compute_slot_mapping(block_tables: Sequence[Sequence[int]], context_lens: Se
     if size < total:
         raise ValueError(f"pad_to={pad_to} is smaller than the {total} tokens of the step")
     gpu = device is not None and torch.device(device).type == "cuda"
+    if gpu and 0 < size <= 0x7fffffff and type(block_size) is int and 0 < block_size <= 0x7fffffff:
+        on_device = _slot_mapping_on_device(block_tables, context_lens, query_lens, block_size, size, device)
+        if on_device is not None:
+            return on_device
     out = torch.empty(size, dtype=torch.long, pin_memory=gpu)
     slots = out.numpy()
     slots[total:] = -1

@@ -32,6 +32,7 @@
 #include "emm_append.inc"
 #include "emm_append_paged.inc"
 #include "emm_concat.inc"
+#include "emm_slots.inc"
 
 namespace {
 int unpack_dequant(void *const *layer_ptrs, int num_layers, int64_t num_blocks,
@@ -326,6 +327,43 @@ int emm_reshape_and_cache_paged_layers(const void *const *key_ptrs, const void *
                       num_tokens, num_heads, head_size, block_size, num_blocks, key_stride_elems,
                       value_stride_elems, src_dtype, cache_elem_bytes, k_scales, v_scales, as_stream(stream),
                       "emm_reshape_and_cache_paged_layers");
+}
+
+int emm_slot_mapping(const int64_t *host_starts, const int64_t *host_offsets, const int64_t *host_first_blocks, int seqs,
+                     const int64_t *host_blocks, int64_t num_blocks, int block_size, int64_t pad_to, int64_t *out,
+                     emm_stream_t stream) {
+  const char *what = "emm_slot_mapping";
+  if (seqs < 0 || num_blocks < 0 || block_size <= 0 || pad_to < 0) return fail(EMM_EINVAL, "%s: negative size", what);
+  if (3 * (int64_t)seqs + 1 + num_blocks > kSlotWords)
+    return fail(EMM_EINVAL, "%s: %d sequences with %lld blocks exceed %d words", what, seqs, (long long)num_blocks, kSlotWords);
+  if (!host_starts || !out || (seqs > 0 && (!host_offsets || !host_first_blocks || !host_blocks)))
+    return fail(EMM_EINVAL, "%s: null pointer", what);
+  SlotTables t;
+  int64_t longest = pad_to - host_starts[seqs];
+  for (int i = 0; i < seqs; ++i) {
+    const int64_t q = host_starts[i + 1] - host_starts[i], off = host_offsets[i], first = host_first_blocks[i];
+    // every block the kernel reads and every slot it writes lies inside what was passed
+    if (host_starts[i] < 0 || q <= 0 || off < 0 || off >= block_size || first < 0 ||
+        first + (off + q - 1) / block_size >= num_blocks)
+      return fail(EMM_EINVAL, "%s: sequence %d does not fit its blocks", what, i);
+    if (q > longest) longest = q;
+    t.word[i] = (uint32_t)host_starts[i];
+    t.word[seqs + i] = (uint32_t)(3 * seqs + 1 + first);
+    t.word[2 * seqs + i] = (uint32_t)off;
+  }
+  if (host_starts[seqs] < 0 || host_starts[seqs] > 0x7fffffffLL || pad_to > 0x7fffffffLL)
+    return fail(EMM_EINVAL, "%s: too many tokens", what);
+  t.word[3 * seqs] = (uint32_t)host_starts[seqs];
+  for (int64_t b = 0; b < num_blocks; ++b) {
+    if (host_blocks[b] < 0 || host_blocks[b] > 0xffffffffLL) return fail(EMM_EINVAL, "%s: block id out of range", what);
+    t.word[3 * seqs + 1 + b] = (uint32_t)host_blocks[b];
+  }
+  const bool pad = pad_to > host_starts[seqs];
+  if (seqs == 0 && !pad) return EMM_OK;
+  const int64_t strips = (longest + 255) / 256;
+  emm_slot_mapping_kernel<<<dim3((uint32_t)(seqs + (pad ? 1 : 0)), (uint32_t)(strips < 64 ? strips : 64)), 256, 0, as_stream(stream)>>>(
+      out, (uint32_t)seqs, (uint32_t)block_size, (uint32_t)pad_to, t);
+  return check_launch(what);
 }
 
 int emm_concat_rows(const void *const *srcs, const int64_t *nbytes, int n, void *dst,

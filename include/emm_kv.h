@@ -45,6 +45,7 @@ extern "C" {
 #define EMM_MAX_INLINE_IDS 512 /* block ids carried by one launch of emm_kv_*_host_ids (longer tables: several launches) */
 #define EMM_MAX_INLINE_PAIRS 480 /* (source, destination) ids carried by one launch of emm_kv_migrate_host_ids */
 #define EMM_MAX_INLINE_PAIRS_TABLES 112 /* the same for pools whose planes are not equally spaced */
+#define EMM_MAX_SLOT_WORDS 960 /* 3 * sequences + 1 + block ids carried by one launch of emm_slot_mapping */
 
 /* error codes */
 #define EMM_OK 0
@@ -357,6 +358,19 @@ int emm_reshape_and_cache_paged_layers(const void *const *key_ptrs,
                                        const float *k_scales,
                                        const float *v_scales,
                                        emm_stream_t stream);
+
+/*
+ * slot mapping of a step from HOST block tables, as vLLM's prepare_model_input derives it from the block tables the
+ * reference passes in SequenceGroupMetadata.block_tables (elasticmm/engine/v0/worker_steps.py:186-218). Sequence i
+ * fills out[host_starts[i] .. host_starts[i + 1]) (host_starts has seqs + 1 entries, each sequence at least one token);
+ * its first token lies at offset host_offsets[i] of block host_blocks[host_first_blocks[i]], the following ones in the
+ * blocks behind it: out = block * block_size + offset. out[host_starts[seqs] .. pad_to) becomes -1. The tables travel in
+ * the kernel argument block: 3 * seqs + 1 + num_blocks <= EMM_MAX_SLOT_WORDS.
+ */
+int emm_slot_mapping(const int64_t *host_starts, const int64_t *host_offsets,
+                     const int64_t *host_first_blocks, int seqs,
+                     const int64_t *host_blocks, int64_t num_blocks, int block_size,
+                     int64_t pad_to, int64_t *out, emm_stream_t stream);
 
 /*
  * concat_rows — copy n ragged segments back to back into `dst`: segment i is

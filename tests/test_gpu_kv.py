@@ -1304,6 +1304,30 @@ def test_paged_append_every_dispatched_wave_shape(cache, H, D, bs, T, phase):
     assert same_bits(kc_g, kc) and same_bits(vc_g, vc)
 
 
+@pytest.mark.parametrize("bs,seqs,chunk,pad", [(16, 1, 0, 0), (16, 24, 0, 3), (16, 239, 0, 0), (16, 240, 0, 0), (12, 400, 1000, 7),
+                                               (16, 0, 16 * 956, 0), (16, 0, 16 * 956 + 1, 5), (16, 30, 8192, 300), (1, 5, 700, 0),
+                                               (16, 1200, 40, 0), (256, 3, 5000, 1)])
+def test_slot_mapping_on_the_device(bs, seqs, chunk, pad):
+    """The kernel's slots (tables in the argument block, one launch to four, longer ones copied) against the host's."""
+    say(f"slot mapping: bs={bs} seqs={seqs} chunk={chunk} pad={pad}")
+    g = torch.Generator().manual_seed(seqs + chunk)
+    lengths = [1] * seqs + [0] * (seqs > 0) + ([chunk] if chunk else [])
+    tables, contexts = [], []
+    for q in lengths:
+        ctx = int(torch.randint(0, 5 * bs, (1,), generator=g))
+        tables.append(torch.randint(0, 2 ** 31, ((ctx + q + bs - 1) // bs + 1,), generator=g).tolist())
+        contexts.append(ctx if q == 1 else ctx % bs * (bs > 1 and chunk % bs != 0))
+    total = sum(lengths)
+    want = cache_ops.compute_slot_mapping(tables, contexts, lengths, bs, pad_to=total + pad)
+    got = cache_ops.compute_slot_mapping(tables, contexts, lengths, bs, pad_to=total + pad, device=torch.device(DEV))
+    assert got.is_cuda and got.dtype == torch.long and torch.equal(got.cpu(), want)
+    if seqs:
+        with pytest.raises(IndexError):
+            cache_ops.compute_slot_mapping([[1, 2]], [2 * bs], [1], bs, device=torch.device(DEV))
+        for other in ([np.array(t) for t in tables], [tuple(t) for t in tables]):  # the general path
+            assert torch.equal(cache_ops.compute_slot_mapping(other, contexts, lengths, bs, pad_to=total + pad, device=DEV).cpu(), want)
+
+
 @pytest.mark.parametrize("layout", ["flash", "paged"])
 @pytest.mark.parametrize("cache", ["auto", "fp8", "fp8_sat"])
 def test_native_append_takes_the_usual_calls_only(layout, cache):
