@@ -1328,6 +1328,38 @@ def test_slot_mapping_on_the_device(bs, seqs, chunk, pad):
             assert torch.equal(cache_ops.compute_slot_mapping(other, contexts, lengths, bs, pad_to=total + pad, device=DEV).cpu(), want)
 
 
+@pytest.mark.parametrize("T", [1, 5, 1536, 1537, 3072, 3073])
+@pytest.mark.parametrize("cache,H,D", [("auto", 4, 128), ("auto", 8, 128), ("auto", 1, 8), ("auto", 5, 104), ("fp8", 4, 128),
+                                       ("fp8", 5, 104), ("fp8_sat", 1, 8), ("fp8_sat", 9, 120), ("fp8", 7, 72)])
+def test_flash_append_on_both_sides_of_its_launch_rules(cache, H, D, T):
+    """Per layer: rows per wave and store policy change past 1536 and 3072 tokens and with rows longer than 1 KiB; fp8 rows
+    of at most 512 elements take the thin waves."""
+    NB, bs = 250, 16
+    g = torch.Generator().manual_seed(T + H)
+    wide = (torch.randn((T, 2 * H * D), generator=g) * 20).to(torch.bfloat16)
+    key, value = (wide[:, i * H * D:(i + 1) * H * D].reshape(T, H, D).contiguous() for i in range(2))
+    slots = torch.randperm(NB * bs, generator=g)[:T]
+    slots[3::17] = -1
+    slots[4::29] = NB * bs + 3  # past the cache: skipped
+    kc = torch.full((NB, bs, H, D), 5, dtype=torch.bfloat16 if cache == "auto" else torch.uint8)
+    vc = kc.clone()
+    kc_g, vc_g, wide_g = kc.to(DEV), vc.to(DEV), wide.to(DEV)
+    key_g, value_g = (wide_g[:, i * H * D:(i + 1) * H * D].view(T, H, D) for i in range(2))
+    inside = torch.where(slots < NB * bs, slots, -1)
+    if cache == "auto":
+        cache_ops.reshape_and_cache_flash(key_g, value_g, kc_g, vc_g, slots.to(DEV))
+        orc.c_reshape_and_cache(key, value, kc, vc, inside)
+    else:
+        ks, vs = torch.tensor([0.05]), torch.tensor([0.11])
+        cache_ops.reshape_and_cache_flash(key_g, value_g, kc_g, vc_g, slots.to(DEV), cache, ks.to(DEV), vs.to(DEV))
+        if cache == "fp8_sat":
+            k8, v8 = (torch.from_numpy(orc.c_quant_fp8_sat(x, float(sc)).reshape(T, H, D).copy()) for x, sc in ((key, ks), (value, vs)))
+            orc.c_reshape_and_cache(k8, v8, kc, vc, inside)
+        else:
+            orc.c_reshape_and_cache_fp8(key, value, kc, vc, inside, float(ks), float(vs))
+    assert same_bits(kc_g, kc) and same_bits(vc_g, vc)
+
+
 @pytest.mark.parametrize("layout", ["flash", "paged"])
 @pytest.mark.parametrize("cache", ["auto", "fp8", "fp8_sat"])
 def test_native_append_takes_the_usual_calls_only(layout, cache):
