@@ -8,6 +8,7 @@ from __future__ import annotations
 import ctypes
 import importlib.util
 import os
+import sys
 from ctypes import c_char_p, c_float, c_int, c_int64, c_void_p, POINTER
 
 from .build import frontend_path, hooks_library_path, library_path
@@ -87,8 +88,10 @@ _frontend_module = None
 
 def _bind_frontend(lib: ctypes.CDLL) -> None:
     """``lib.frontend``: the native host side of the per-layer appends (csrc/emm_frontend.cpp) over this library's
-    entry points."""
+    entry points. Without torch there are no tensors to check and only the C ABI is bound."""
     global _frontend_module
+    if "torch" not in sys.modules:
+        return
     if _frontend_module is None:
         path = frontend_path()
         if not os.path.exists(path):
@@ -115,7 +118,10 @@ def load() -> ctypes.CDLL:
             "(run `python -m elasticmm_amd.build`). There is no CPU fallback.")
     # torch carries its own copy of the HIP runtime and exports its symbols globally. Streams and device pointers
     # come from torch, so the library has to bind to that copy: torch is loaded before the library is.
-    import torch  # noqa: F401
+    try:
+        import torch  # noqa: F401
+    except ImportError:
+        pass
     lib = ctypes.CDLL(path)
     for name, (res, args) in SIGNATURES.items():
         fn = getattr(lib, name)  # AttributeError if the symbol is not exported
@@ -137,7 +143,10 @@ def load_hooks() -> ctypes.CDLL:
     path = hooks_library_path()
     if not os.path.exists(path):
         raise RuntimeError(f"{path} is missing (run `python -m elasticmm_amd.build`)")
-    import torch  # noqa: F401
+    try:
+        import torch  # noqa: F401
+    except ImportError:
+        pass
     lib = ctypes.CDLL(path)
     for name, (res, args) in {**SIGNATURES, **HOOK_SIGNATURES}.items():
         fn = getattr(lib, name)

@@ -113,12 +113,14 @@ PyObject *frontend_flash(PyObject *self, PyObject *const *args, Py_ssize_t nargs
     if (c.kc->numel() % row || c.vc->numel() != c.kc->numel()) return not_usual();
     const int64_t eb = c.key->element_size();
     const int64_t *map = static_cast<const int64_t *>(c.slots->data_ptr());
+    const void *key = c.key->data_ptr(), *value = c.value->data_ptr();
+    void *kc = c.kc->data_ptr(), *vc = c.vc->data_ptr();
+    Py_BEGIN_ALLOW_THREADS // a launch may wait for room in the stream's queue; the caller's frame holds the tensors
     if (mode == kAuto)
-      rc = f->append(c.key->data_ptr(), c.value->data_ptr(), c.kc->data_ptr(), c.vc->data_ptr(), map, T, row * eb, ks * eb,
-                     vs * eb, slots, c.stream);
+      rc = f->append(key, value, kc, vc, map, T, row * eb, ks * eb, vs * eb, slots, c.stream);
     else
-      rc = f->append_fp8(c.key->data_ptr(), c.value->data_ptr(), c.kc->data_ptr(), c.vc->data_ptr(), map, T, row, ks, vs,
-                         slots, c.k_scale, c.v_scale, c.src_dtype, c.stream);
+      rc = f->append_fp8(key, value, kc, vc, map, T, row, ks, vs, slots, c.k_scale, c.v_scale, c.src_dtype, c.stream);
+    Py_END_ALLOW_THREADS
   } catch (const std::exception &) { // a tensor that could not be looked at: the Python operator says why
     return not_usual();
   }
@@ -138,9 +140,13 @@ PyObject *frontend_paged(PyObject *self, PyObject *const *args, Py_ssize_t nargs
     if (c.vc->size(0) != NB || c.vc->size(1) != H || c.vc->size(2) != D || c.vc->size(3) != bs) return not_usual();
     const int64_t ks = token_stride(*c.key), vs = token_stride(*c.value);
     if (ks < H * D || vs < H * D || H > INT_MAX || D > INT_MAX || bs > INT_MAX) return not_usual();
-    rc = f->append_paged(c.key->data_ptr(), c.value->data_ptr(), c.kc->data_ptr(), c.vc->data_ptr(),
-                         static_cast<const int64_t *>(c.slots->data_ptr()), T, (int)H, (int)D, (int)bs, NB, ks, vs,
-                         c.src_dtype, (int)ceb, c.k_scale, c.v_scale, c.stream);
+    const int64_t *map = static_cast<const int64_t *>(c.slots->data_ptr());
+    const void *key = c.key->data_ptr(), *value = c.value->data_ptr();
+    void *kc = c.kc->data_ptr(), *vc = c.vc->data_ptr();
+    Py_BEGIN_ALLOW_THREADS // as above
+    rc = f->append_paged(key, value, kc, vc, map, T, (int)H, (int)D, (int)bs, NB, ks, vs, c.src_dtype, (int)ceb, c.k_scale,
+                         c.v_scale, c.stream);
+    Py_END_ALLOW_THREADS
   } catch (const std::exception &) {
     return not_usual();
   }
