@@ -334,31 +334,33 @@ int emm_slot_mapping(const int64_t *host_starts, const int64_t *host_offsets, co
                      emm_stream_t stream) {
   const char *what = "emm_slot_mapping";
   if (seqs < 0 || num_blocks < 0 || block_size <= 0 || pad_to < 0) return fail(EMM_EINVAL, "%s: negative size", what);
-  if (3 * (int64_t)seqs + 1 + num_blocks > kSlotWords)
+  if (num_blocks > kSlotWords || 3 * (int64_t)seqs + 1 + num_blocks > kSlotWords)
     return fail(EMM_EINVAL, "%s: %d sequences with %lld blocks exceed %d words", what, seqs, (long long)num_blocks, kSlotWords);
   if (!host_starts || !out || (seqs > 0 && (!host_offsets || !host_first_blocks || !host_blocks)))
     return fail(EMM_EINVAL, "%s: null pointer", what);
+  const int64_t total = host_starts[seqs];
+  if (total < 0 || total > 0x7fffffffLL || pad_to > 0x7fffffffLL) return fail(EMM_EINVAL, "%s: too many tokens", what);
+  if (pad_to < total)
+    return fail(EMM_EINVAL, "%s: pad_to=%lld (the size of out) is smaller than the %lld tokens", what, (long long)pad_to, (long long)total);
   SlotTables t;
-  int64_t longest = pad_to - host_starts[seqs];
+  int64_t longest = pad_to - total;
   for (int i = 0; i < seqs; ++i) {
-    const int64_t q = host_starts[i + 1] - host_starts[i], off = host_offsets[i], first = host_first_blocks[i];
-    // every block the kernel reads and every slot it writes lies inside what was passed
-    if (host_starts[i] < 0 || q <= 0 || off < 0 || off >= block_size || first < 0 ||
-        first + (off + q - 1) / block_size >= num_blocks)
+    const int64_t start = host_starts[i], end = host_starts[i + 1], off = host_offsets[i], first = host_first_blocks[i];
+    // every block the kernel reads lies inside the words, every slot it writes inside out[0 .. pad_to)
+    if (start < 0 || end <= start || end > total || off < 0 || off >= block_size || first < 0 || first >= num_blocks ||
+        (off + (end - start) - 1) / block_size >= num_blocks - first)
       return fail(EMM_EINVAL, "%s: sequence %d does not fit its blocks", what, i);
-    if (q > longest) longest = q;
-    t.word[i] = (uint32_t)host_starts[i];
+    if (end - start > longest) longest = end - start;
+    t.word[i] = (uint32_t)start;
     t.word[seqs + i] = (uint32_t)(3 * seqs + 1 + first);
     t.word[2 * seqs + i] = (uint32_t)off;
   }
-  if (host_starts[seqs] < 0 || host_starts[seqs] > 0x7fffffffLL || pad_to > 0x7fffffffLL)
-    return fail(EMM_EINVAL, "%s: too many tokens", what);
-  t.word[3 * seqs] = (uint32_t)host_starts[seqs];
+  t.word[3 * seqs] = (uint32_t)total;
   for (int64_t b = 0; b < num_blocks; ++b) {
     if (host_blocks[b] < 0 || host_blocks[b] > 0xffffffffLL) return fail(EMM_EINVAL, "%s: block id out of range", what);
     t.word[3 * seqs + 1 + b] = (uint32_t)host_blocks[b];
   }
-  const bool pad = pad_to > host_starts[seqs];
+  const bool pad = pad_to > total;
   if (seqs == 0 && !pad) return EMM_OK;
   const int64_t strips = (longest + 255) / 256;
   emm_slot_mapping_kernel<<<dim3((uint32_t)(seqs + (pad ? 1 : 0)), (uint32_t)(strips < 64 ? strips : 64)), 256, 0, as_stream(stream)>>>(

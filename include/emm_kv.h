@@ -364,8 +364,9 @@ int emm_reshape_and_cache_paged_layers(const void *const *key_ptrs,
  * reference passes in SequenceGroupMetadata.block_tables (elasticmm/engine/v0/worker_steps.py:186-218). Sequence i
  * fills out[host_starts[i] .. host_starts[i + 1]) (host_starts has seqs + 1 entries, each sequence at least one token);
  * its first token lies at offset host_offsets[i] of block host_blocks[host_first_blocks[i]], the following ones in the
- * blocks behind it: out = block * block_size + offset. out[host_starts[seqs] .. pad_to) becomes -1. The tables travel in
- * the kernel argument block: 3 * seqs + 1 + num_blocks <= EMM_MAX_SLOT_WORDS.
+ * blocks behind it: out = block * block_size + offset. out[host_starts[seqs] .. pad_to) becomes -1: `out` holds pad_to
+ * slots, and pad_to smaller than host_starts[seqs] is EMM_EINVAL. The tables travel in the kernel argument block:
+ * 3 * seqs + 1 + num_blocks <= EMM_MAX_SLOT_WORDS. `out` and `stream` belong to the current device.
  */
 int emm_slot_mapping(const int64_t *host_starts, const int64_t *host_offsets,
                      const int64_t *host_first_blocks, int seqs,

@@ -112,6 +112,43 @@ def test_argument_errors_of_the_layout_variants_without_gpu():
     assert lib.emm_reshape_and_cache_strided(t, t, t, t, 0, P, 4, 2, 64, 16, 8, 128, 128, 4096, 128, 64, None) == 0
 
 
+def test_argument_errors_of_the_slot_mapping_without_gpu():
+    """Whatever would make the kernel read past its words or write past `out` is refused before the launch."""
+    import numpy as np
+
+    lib = _lib.load()
+    P, MAX = 0x1000, 2 ** 63 - 1
+
+    def call(starts, offsets, firsts, blocks, bs=16, pad_to=None, out=P, seqs=None, num_blocks=None):
+        a = [np.array(x, dtype=np.int64) for x in (starts, offsets, firsts, blocks)]
+        return lib.emm_slot_mapping(a[0].ctypes.data, a[1].ctypes.data, a[2].ctypes.data, len(offsets) if seqs is None else seqs,
+                                    a[3].ctypes.data, len(blocks) if num_blocks is None else num_blocks, bs,
+                                    starts[-1] if pad_to is None else pad_to, out, None)
+
+    def refused(text, *args, **kw):
+        assert call(*args, **kw) == -1 and text in lib.emm_last_error(), (args, kw, lib.emm_last_error())
+
+    for kw in ({"seqs": -1}, {"num_blocks": -1}, {"bs": 0}, {"pad_to": -1}):
+        refused(b"negative size", [0, 100], [0], [0], [1] * 7, **kw)
+    # `pad_to` is the size of `out`: never smaller than the tokens the sequences have
+    refused(b"smaller than", [0, 100], [0], [0], [1] * 7, pad_to=99)
+    refused(b"smaller than", [0, 100], [0], [0], [1] * 7, pad_to=0)
+    refused(b"null pointer", [0, 100], [0], [0], [1] * 7, out=None)
+    # counts of which the sum does not fit 64 bits
+    refused(b"exceed", [0, 100], [0], [0], [1] * 7, num_blocks=MAX)
+    refused(b"exceed", [0, 100], [0], [0], [1] * 7, seqs=2 ** 31 - 1)
+    refused(b"exceed", [0, 1], [0], [0], [1] * (_lib.EMM_MAX_SLOT_WORDS - 3))
+    for starts, off, first in (([0, 100], 0, 1), ([0, 100], 13, 0), ([0, 17], 0, MAX), ([0, 1], 0, 7), ([0, 1], 16, 0), ([0, 1], -1, 0),
+                               ([0, 1], 0, -1), ([0, 0], 0, 0), ([5, 4], 0, 0), ([-1, 1], 0, 0), ([0, 2 ** 31], 0, 0),
+                               ([0, MAX], 15, 0), ([MAX, -MAX - 1], 0, 0)):
+        refused(b"", starts, [off], [first], [1] * 7, pad_to=max(0, starts[-1]))
+    refused(b"too many tokens", [0], [], [], [], pad_to=2 ** 31)
+    refused(b"too many tokens", [-1], [], [], [], pad_to=5)
+    refused(b"block id", [0, 1], [0], [0], [-1])
+    refused(b"block id", [0, 1], [0], [0], [2 ** 32])
+    assert call([0], [], [], []) == 0  # nothing to write: never reaches the device
+
+
 def test_last_error_is_kept_per_thread():
     """Two host threads that fail in different ways each read their own message (the text lives in
     thread-local storage; the transfer manager calls the library from a thread of its own)."""
