@@ -30,6 +30,16 @@ def _stream_ptr(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+_get_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
+def _elsewhere(device: torch.device) -> bool:
+    """True if ``device`` is not the GPU that is current: a launch then has to be made under
+    ``torch.cuda.device(device)``. The default stream's handle is null on every GPU, and a null stream is the one of
+    the current GPU: the kernel would run there, on memory of another one and beside that one's streams."""
+    return device.index is not None and device.index != _get_device()
+
+
 def _require_gpu(t: torch.Tensor, what: str) -> None:
     if not t.is_cuda:
         raise RuntimeError(f"{what}: tensor is on {t.device}; the KV kernels run on the GPU only")

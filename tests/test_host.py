@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 import torch
 
-from elasticmm_amd import kv_ops
+from elasticmm_amd import _lib, cache_ops, kv_ops
 from elasticmm_amd.block_manager import BlockLocation, BlockManager, VisionBlockManager
 from elasticmm_amd.kv_transfer import KVTransferManager, TransferMethod
 from elasticmm_amd.worker import KVWorker, LoopbackLink
@@ -649,3 +649,61 @@ def test_compute_slot_mapping_matches_the_definition():
         cache_ops.compute_slot_mapping([[1, 2]], [0], [20], 16, pad_to=8)
     with pytest.raises(ValueError, match="differ in length"):
         cache_ops.compute_slot_mapping([[1]], [0, 1], [1], 16)
+
+
+class OtherGpuIsCurrent:
+    """GPU 0 is current and everything lives on GPU 1, without a GPU: which device is current is kept here, the library
+    is a stub that records it for every entry point that is called, and new tensors are CPU memory that claims GPU 1."""
+
+    def __init__(self, monkeypatch):
+        self.current, self.calls = 0, []
+        rig = self
+
+        class Device:
+            def __init__(self, device):
+                self.index = torch.device(device).index
+
+            def __enter__(self):
+                self.back, rig.current = rig.current, self.index
+
+            def __exit__(self, *exc):
+                rig.current = self.back
+
+        class Lib:
+            def __getattr__(self, name):
+                def entry(*args):
+                    rig.calls.append((name, rig.current))
+                    return 0
+                return entry
+
+        monkeypatch.setattr(torch.cuda, "device", Device)
+        monkeypatch.setattr(kv_ops, "_get_device", lambda: rig.current)
+        monkeypatch.setattr(kv_ops, "_raw_stream", lambda index: 0)
+        monkeypatch.setattr(_lib, "_lib", Lib())
+        real_empty = torch.empty
+        monkeypatch.setattr(torch, "empty", lambda *a, **kw: OnGpu1(real_empty(*a, **{**kw, "device": "cpu"}))
+                            if "device" in kw else real_empty(*a, **kw))
+
+    def launched_on_1(self, *names):
+        got, self.calls = self.calls, []
+        assert self.current == 0, "the current device was not put back"
+        assert got and {n for n, _ in got} == set(names) and {d for _, d in got} == {1}, got
+
+
+class OnGpu1:
+    """A CPU tensor that says it lies on GPU 1."""
+    is_cuda, device = True, torch.device("cuda:1")
+
+    def __init__(self, t):
+        self._t = t
+
+    def __getattr__(self, name):
+        return getattr(self._t, name)
+
+
+def test_slot_mapping_is_launched_on_the_gpu_it_is_for(monkeypatch):
+    """A null stream is the current GPU's: a step's slots for GPU 1 must not be written by a kernel on GPU 0."""
+    rig = OtherGpuIsCurrent(monkeypatch)
+    got = cache_ops.compute_slot_mapping([[3], [1, 2]], [5, 0], [1, 20], 16, pad_to=24, device="cuda:1")
+    assert got.numel() == 24
+    rig.launched_on_1("emm_slot_mapping")
