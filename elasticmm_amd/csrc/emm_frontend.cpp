@@ -13,6 +13,8 @@
 #include <Python.h>
 #include <ATen/ATen.h>
 #include <ATen/TensorSubclassLikeUtils.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -88,6 +90,12 @@ bool take(PyObject *const *args, Py_ssize_t nargs, Call &c, int &mode) {
   return true;
 }
 
+// The launch goes to the current device whatever the stream (the default stream's handle is null on every device):
+// the tensors' device has to be current.
+void make_current(const Call &c, c10::OptionalDeviceGuard &guard) {
+  if (c10::hip::current_device() != c.key->device().index()) guard.reset_device(c.key->device());
+}
+
 PyObject *not_usual() { return PyLong_FromLong(0); }
 
 // A refused call (EMM_EINVAL comes before any launch) goes to the Python operator, which reports it.
@@ -115,6 +123,8 @@ PyObject *frontend_flash(PyObject *self, PyObject *const *args, Py_ssize_t nargs
     const int64_t *map = static_cast<const int64_t *>(c.slots->data_ptr());
     const void *key = c.key->data_ptr(), *value = c.value->data_ptr();
     void *kc = c.kc->data_ptr(), *vc = c.vc->data_ptr();
+    c10::OptionalDeviceGuard guard;
+    make_current(c, guard);
     Py_BEGIN_ALLOW_THREADS // a launch may wait for room in the stream's queue; the caller's frame holds the tensors
     if (mode == kAuto)
       rc = f->append(key, value, kc, vc, map, T, row * eb, ks * eb, vs * eb, slots, c.stream);
@@ -143,6 +153,8 @@ PyObject *frontend_paged(PyObject *self, PyObject *const *args, Py_ssize_t nargs
     const int64_t *map = static_cast<const int64_t *>(c.slots->data_ptr());
     const void *key = c.key->data_ptr(), *value = c.value->data_ptr();
     void *kc = c.kc->data_ptr(), *vc = c.vc->data_ptr();
+    c10::OptionalDeviceGuard guard;
+    make_current(c, guard);
     Py_BEGIN_ALLOW_THREADS // as above
     rc = f->append_paged(key, value, kc, vc, map, T, (int)H, (int)D, (int)bs, NB, ks, vs, c.src_dtype, (int)ceb, c.k_scale,
                          c.v_scale, c.stream);

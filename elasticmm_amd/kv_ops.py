@@ -20,17 +20,14 @@ from ._lib import (EMM_DTYPE_BF16, EMM_DTYPE_F16, EMM_FP8_SATURATE, EMM_MAX_INLI
 IndexLike = Union[Sequence[int], np.ndarray, torch.Tensor]
 
 
-_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+# the current GPU's index, and the hipStream_t of torch's current stream on a GPU given by its index
+_get_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", lambda index: torch.cuda.current_stream(index).cuda_stream)
 
 
 def _stream_ptr(device: torch.device) -> int:
     """hipStream_t of torch's current stream on `device`, as an integer."""
-    if _raw_stream is not None and device.index is not None:
-        return _raw_stream(device.index)
-    return torch.cuda.current_stream(device).cuda_stream
-
-
-_get_device = getattr(torch._C, "_cuda_getDevice", None)
+    return _raw_stream(device.index if device.index is not None else _get_device())
 
 
 def _elsewhere(device: torch.device) -> bool:
@@ -137,6 +134,7 @@ class PoolView:
                 raise ValueError(f"layer {i} is not contiguous")
         self.layers: List[torch.Tensor] = layers
         self.device = first.device if pinned_host_for is None else torch.device(pinned_host_for)
+        self.gpu = self.device.index  # None: whichever is current
         self.on_host = pinned_host_for is not None
         self.dtype = first.dtype
         self.elem_bytes = first.element_size()
@@ -218,13 +216,17 @@ def kv_pack(pool: PoolView, block_indices: IndexLike, out: Optional[torch.Tensor
     the allocation held. ``strict=True`` validates a device table first (``check_device_block_ids``: one
     reduction and a synchronisation) and raises ``IndexError`` instead."""
     lib = _lib.load()
+    here = _get_device()  # (_elsewhere, spelt out: this runs in front of kernels of a few microseconds)
+    if pool.gpu != here and pool.gpu is not None:
+        with torch.cuda.device(pool.device):
+            return kv_pack(pool, block_indices, out, strict)
     n, table_arg, inline, keep = _table_for_launch(block_indices, pool, strict, "kv_pack")
     if out is None:
         out = torch.empty((pool.num_layers, pool.num_kv, n) + pool.block_shape, dtype=pool.dtype, device=pool.device)
     elif out.device != pool.device or out.dtype != pool.dtype or not out.is_contiguous() \
             or out.numel() != pool.num_layers * pool.num_kv * n * pool.chunk_elems:
         raise ValueError("kv_pack: `out` must be a contiguous pool-dtype tensor of the packed size")
-    stream = _stream_ptr(pool.device)
+    stream = _raw_stream(here)
     plane = pool.num_kv * n * pool.chunk_bytes
     fn = lib.emm_kv_pack_host_ids if inline else lib.emm_kv_pack
     base = out.data_ptr()
@@ -242,6 +244,10 @@ def kv_unpack(pool: PoolView, block_indices: IndexLike, packed: torch.Tensor, st
     lib = _lib.load()
     if not packed.is_cuda:
         _require_gpu(packed, "kv_unpack")
+    here = _get_device()  # (_elsewhere, spelt out: this runs in front of kernels of a few microseconds)
+    if pool.gpu != here and pool.gpu is not None:
+        with torch.cuda.device(pool.device):
+            return kv_unpack(pool, block_indices, packed, strict)
     n, table_arg, inline, keep = _table_for_launch(block_indices, pool, strict, "kv_unpack")
     if packed.device != pool.device:
         raise ValueError("kv_unpack: packed buffer is on another device")
@@ -251,7 +257,7 @@ def kv_unpack(pool: PoolView, block_indices: IndexLike, packed: torch.Tensor, st
                          f"pool geometry needs {pool.num_layers * pool.num_kv * n * pool.chunk_bytes}")
     if not packed.is_contiguous():
         packed = packed.contiguous()
-    stream = _stream_ptr(pool.device)
+    stream = _raw_stream(here)
     plane = pool.num_kv * n * pool.chunk_bytes
     fn = lib.emm_kv_unpack_host_ids if inline else lib.emm_kv_unpack
     base = packed.data_ptr()
@@ -267,6 +273,9 @@ def kv_migrate(src: PoolView, src_indices: IndexLike, dst: PoolView, dst_indices
     """``dst[l][:, dst_idx[j]] = src[l][:, src_idx[j]]`` in one launch, no staging buffer (``strict``: as in
     ``kv_pack``, for either table)."""
     lib = _lib.load()
+    if _elsewhere(src.device):
+        with torch.cuda.device(src.device):
+            return kv_migrate(src, src_indices, dst, dst_indices, strict)
     if strict:
         for idx, pool, what in ((src_indices, src, "kv_migrate (source table)"), (dst_indices, dst, "kv_migrate (destination table)")):
             if isinstance(idx, torch.Tensor) and idx.is_cuda:
@@ -303,6 +312,9 @@ def copy_blocks(pool: PoolView, block_mapping: Union[torch.Tensor, Sequence[Sequ
     """All layers: ``pool[:, dst] = pool[:, src]`` for the (src, dst) rows of ``block_mapping`` (``strict``: a
     device mapping is validated first, as in ``kv_pack``; without it pairs with an id out of range are skipped)."""
     lib = _lib.load()
+    if _elsewhere(pool.device):
+        with torch.cuda.device(pool.device):
+            return copy_blocks(pool, block_mapping, strict)
     if strict and isinstance(block_mapping, torch.Tensor) and block_mapping.is_cuda:
         check_device_block_ids(block_mapping, pool.num_blocks, "copy_blocks")
     if isinstance(block_mapping, torch.Tensor):
@@ -344,6 +356,9 @@ def kv_unpack_dequant_fp8(pool: PoolView, block_indices: IndexLike, packed_fp8: 
     """Scatter an fp8-e4m3fn transfer buffer ``[L, 2, n, ...]`` into a bf16/f16 pool,
     ``out = rne16(float(q) * scale)`` with per-layer K and V scales."""
     lib = _lib.load()
+    if _elsewhere(pool.device):
+        with torch.cuda.device(pool.device):
+            return kv_unpack_dequant_fp8(pool, block_indices, packed_fp8, k_scales, v_scales)
     _require_gpu(packed_fp8, "kv_unpack_dequant_fp8")
     if pool.num_kv != 2:
         raise ValueError("kv_unpack_dequant_fp8 needs a [2, num_blocks, ...] pool")
@@ -417,6 +432,9 @@ def reshape_and_cache(key: torch.Tensor, value: torch.Tensor, key_cache: torch.T
     lib = _lib.load()
     if not (key.is_cuda and value.is_cuda and key_cache.is_cuda and value_cache.is_cuda and slot_mapping.is_cuda):
         raise RuntimeError("reshape_and_cache: every tensor must be on the GPU; the KV kernels run on the GPU only")
+    if _elsewhere(key.device):
+        with torch.cuda.device(key.device):
+            return reshape_and_cache(key, value, key_cache, value_cache, slot_mapping, k_scale, v_scale, saturate)
     if slot_mapping.dtype != torch.long:
         raise TypeError("slot_mapping must be int64")
     if not slot_mapping.is_contiguous():
@@ -470,6 +488,9 @@ def reshape_and_cache_strided(keys: Sequence[torch.Tensor], values: Sequence[tor
     k, v, kc, vc = keys[0], values[0], key_caches[0], value_caches[0]
     for t in (k, v, kc, vc):
         _require_gpu(t, "reshape_and_cache_strided")
+    if _elsewhere(k.device):
+        with torch.cuda.device(k.device):
+            return reshape_and_cache_strided(keys, values, key_caches, value_caches, slot_mapping, k_scales, v_scales, saturate)
     if k.dim() != 3 or v.shape != k.shape:
         raise ValueError("key and value must be [num_tokens, num_heads, head_size] of one shape")
     T, H, D = (int(x) for x in k.shape)
@@ -562,6 +583,9 @@ def reshape_and_cache_paged(key: torch.Tensor, value: torch.Tensor, key_cache: t
     16-bit source is quantised to fp8-e4m3fn with ``k_scale`` / ``v_scale``."""
     lib = _lib.load()
     T, H, D, bs, NB, ks, vs, ceb = _paged_geometry(key, value, key_cache, value_cache)
+    if _elsewhere(key.device):
+        with torch.cuda.device(key.device):
+            return reshape_and_cache_paged(key, value, key_cache, value_cache, slot_mapping, k_scale, v_scale, saturate)
     slot_mapping = _check_slot_mapping(slot_mapping, T)
     k_ptr = v_ptr = None
     keep = None
@@ -618,6 +642,9 @@ class PagedLayeredAppend:
     def __call__(self, slot_mapping: torch.Tensor) -> None:
         if self.num_layers == 0:
             return
+        if _elsewhere(self.device):
+            with torch.cuda.device(self.device):
+                return self(slot_mapping)
         T, H, D, bs, NB, ks, vs, ceb = self.geom
         slot_mapping = _check_slot_mapping(slot_mapping, T)
         stream = _stream_ptr(self.device)
@@ -685,6 +712,9 @@ class LayeredAppend:
     def __call__(self, slot_mapping: torch.Tensor) -> None:
         if self.num_layers == 0:
             return
+        if _elsewhere(self.device):
+            with torch.cuda.device(self.device):
+                return self(slot_mapping)
         if slot_mapping.dtype != torch.long or not slot_mapping.is_cuda:
             raise TypeError("slot_mapping must be an int64 GPU tensor")
         if not slot_mapping.is_contiguous():
@@ -713,8 +743,11 @@ def reshape_and_cache_layers(keys: Sequence[torch.Tensor], values: Sequence[torc
     LayeredAppend(keys, values, key_caches, value_caches, k_scales, v_scales, saturate)(slot_mapping)
 
 
-def _launch_concat(lib, ptrs, sizes, out: torch.Tensor, stream) -> None:
-    off = 0
+def _launch_concat(lib, ptrs, sizes, out: torch.Tensor) -> None:
+    if _elsewhere(out.device):
+        with torch.cuda.device(out.device):
+            return _launch_concat(lib, ptrs, sizes, out)
+    stream, off = _stream_ptr(out.device), 0
     for i0 in range(0, len(ptrs), EMM_MAX_SEGMENTS):
         n = min(EMM_MAX_SEGMENTS, len(ptrs) - i0)
         srcs = (_lib.c_void_p * n)(*ptrs[i0:i0 + n])
@@ -756,7 +789,7 @@ def concat_rows(tensors: Sequence[torch.Tensor], out: Optional[torch.Tensor] = N
         out = torch.empty(shape, dtype=dtype, device=device)
     elif tuple(out.shape) != shape or out.dtype != dtype or out.device != device or not out.is_contiguous():
         raise ValueError("concat_rows: `out` has the wrong shape / dtype / device or is not contiguous")
-    _launch_concat(lib, ptrs, sizes, out, _stream_ptr(device))
+    _launch_concat(lib, ptrs, sizes, out)
     del alive  # queued on the stream the copies were made on: the allocator may reuse them now
     return out
 
@@ -800,7 +833,7 @@ def concat_row_sources(sources: Sequence[RowSource], out: Optional[torch.Tensor]
         out = torch.empty(shape, dtype=dtype, device=device)
     elif tuple(out.shape) != shape or out.dtype != dtype or out.device != device or not out.is_contiguous():
         raise ValueError("concat_row_sources: `out` has the wrong shape / dtype / device or is not contiguous")
-    _launch_concat(lib, ptrs, sizes, out, _stream_ptr(device))
+    _launch_concat(lib, ptrs, sizes, out)
     return out
 
 
@@ -808,6 +841,9 @@ def stream_copy(src: torch.Tensor, dst: torch.Tensor) -> None:
     """Plain device copy with the block-move tile engine (benchmark yardstick)."""
     lib = _lib.load()
     _require_gpu(src, "stream_copy")
+    if _elsewhere(src.device):
+        with torch.cuda.device(src.device):
+            return stream_copy(src, dst)
     nbytes = src.numel() * src.element_size()
     if dst.numel() * dst.element_size() != nbytes or not src.is_contiguous() or not dst.is_contiguous():
         raise ValueError("stream_copy: contiguous tensors of equal byte size required")

@@ -1410,6 +1410,25 @@ def test_native_append_takes_the_usual_calls_only(layout, cache):
             assert same_bits(c[0], want[0]) and same_bits(c[1], want[1]), f"odd call {n}"
 
 
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="needs a second GPU")
+@pytest.mark.parametrize("layout", ["flash", "paged"])
+def test_native_append_on_a_gpu_that_is_not_current(layout):
+    """The native host side launches on its tensors' GPU, not on the current one, and leaves the current one as it was."""
+    T, H, D, NB, bs, dev = 40, 2, 64, 6, 16, torch.device("cuda:1")
+    g = torch.Generator().manual_seed(8)
+    key, value = (torch.randn((T, H, D), generator=g).to(torch.bfloat16) for _ in range(2))
+    slots = torch.randperm(NB * bs, generator=g)[:T]
+    shapes = [(NB, bs, H, D)] * 2 if layout == "flash" else [(NB, H, D // 8, bs, 8), (NB, H, D, bs)]
+    want = [torch.zeros(sh, dtype=torch.bfloat16) for sh in shapes]
+    got = [t.to(dev) for t in want]
+    native = getattr(_lib.load().frontend, "append_" + layout)
+    with torch.cuda.device(0):
+        assert native(key.to(dev), value.to(dev), *got, slots.to(dev), 0, None, None) == 1
+        assert torch.cuda.current_device() == 0
+    (orc.c_reshape_and_cache if layout == "flash" else orc.c_reshape_and_cache_paged)(key, value, *want, slots)
+    assert same_bits(got[0], want[0]) and same_bits(got[1], want[1])
+
+
 def test_fp8_append_exhaustive_bf16_and_f16(golden_dir):
     """Every 16-bit input x several scales through the append kernel: 64 tokens x 1024
     elements is exactly the 65 536 bit patterns."""

@@ -1,4 +1,6 @@
 """Host-side logic of the drop-in surface (no GPU needed)."""
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 import torch
@@ -670,6 +672,8 @@ class OtherGpuIsCurrent:
                 rig.current = self.back
 
         class Lib:
+            frontend = SimpleNamespace(append_flash=lambda *a: 0, append_paged=lambda *a: 0)  # "not a usual call"
+
             def __getattr__(self, name):
                 def entry(*args):
                     rig.calls.append((name, rig.current))
@@ -707,3 +711,50 @@ def test_slot_mapping_is_launched_on_the_gpu_it_is_for(monkeypatch):
     got = cache_ops.compute_slot_mapping([[3], [1, 2]], [5, 0], [1, 20], 16, pad_to=24, device="cuda:1")
     assert got.numel() == 24
     rig.launched_on_1("emm_slot_mapping")
+
+
+def test_every_operator_is_launched_on_its_tensors_gpu(monkeypatch):
+    rig = OtherGpuIsCurrent(monkeypatch)
+    monkeypatch.setattr(kv_ops, "block_index_tensor", lambda ids, nb, dev: torch.as_tensor(np.asarray(ids, dtype=np.int64)))
+    monkeypatch.setattr(kv_ops, "_scales_tensor", lambda scales, n, dev: torch.ones(n))
+    L, NB, bs, H, D, T = 2, 6, 16, 1, 16, 5
+    new = lambda *shape, dtype=torch.bfloat16: OnGpu1(torch.zeros(shape, dtype=dtype))  # noqa: E731
+    pools = [kv_ops.PoolView([new(2, NB, bs, H, D) for _ in range(L)]) for _ in range(2)]
+
+    packed = kv_ops.kv_pack(pools[0], [0, 3])
+    rig.launched_on_1("emm_kv_pack_host_ids")
+    kv_ops.kv_unpack(pools[1], [1, 2], packed)
+    rig.launched_on_1("emm_kv_unpack_host_ids")
+    kv_ops.kv_migrate(pools[0], [0, 3], pools[1], [1, 2])
+    rig.launched_on_1("emm_kv_migrate_host_ids")
+    kv_ops.kv_migrate(pools[0], list(range(NB)) * 200, pools[1], list(range(NB)) * 200)
+    rig.launched_on_1("emm_kv_migrate")
+    kv_ops.copy_blocks(pools[0], [[0, 1]])
+    rig.launched_on_1("emm_copy_blocks")
+    kv_ops.kv_unpack_dequant_fp8(pools[0], [4], new(L, 2, 1, bs, H, D, dtype=torch.uint8), 1.0, 1.0)
+    rig.launched_on_1("emm_kv_unpack_dequant_fp8_host_ids")
+
+    key, slots = new(T, H, D), OnGpu1(torch.arange(T))
+    for cache, fp8 in ((torch.bfloat16, False), (torch.uint8, True)):
+        x = 16 // (1 if fp8 else 2)
+        mode, scales = ("fp8", (1.0, 1.0)) if fp8 else ("auto", ())
+        flat = [new(NB, bs, H, D, dtype=cache) for _ in range(2)]
+        paged = [new(NB, H, D // x, bs, x, dtype=cache), new(NB, H, D, bs, dtype=cache)]
+        headed = [OnGpu1(torch.zeros((NB, H + 1, bs, D), dtype=cache)[:, :H].permute(0, 2, 1, 3)) for _ in range(2)]
+        cache_ops.reshape_and_cache_flash(key, key, *flat, slots, mode, *scales)
+        rig.launched_on_1("emm_reshape_and_cache_fp8" if fp8 else "emm_reshape_and_cache")
+        cache_ops.reshape_and_cache_flash(key, key, *headed, slots, mode, *scales)
+        rig.launched_on_1("emm_reshape_and_cache_strided_fp8" if fp8 else "emm_reshape_and_cache_strided")
+        cache_ops.reshape_and_cache(key, key, *paged, slots, mode, *scales)
+        rig.launched_on_1("emm_reshape_and_cache_paged")
+        kv_ops.LayeredAppend([key] * L, [key] * L, [flat[0]] * L, [flat[1]] * L, *scales)(slots)
+        rig.launched_on_1("emm_reshape_and_cache_fp8_layers" if fp8 else "emm_reshape_and_cache_layers")
+        kv_ops.PagedLayeredAppend([key] * L, [key] * L, [paged[0]] * L, [paged[1]] * L, *scales)(slots)
+        rig.launched_on_1("emm_reshape_and_cache_paged_layers")
+
+    kv_ops.concat_rows([key, key])
+    rig.launched_on_1("emm_concat_rows")
+    kv_ops.concat_row_sources([kv_ops.RowSource(key)])
+    rig.launched_on_1("emm_concat_rows")
+    kv_ops.stream_copy(key, new(T, H, D))
+    rig.launched_on_1("emm_stream_copy")
