@@ -187,9 +187,38 @@ def swap_blocks(src_kv_cache: torch.Tensor, dst_kv_cache: torch.Tensor, src_to_d
 _MAX_SLOT_LAUNCHES = 4
 
 
-def _slot_mapping_on_device(block_tables, context_lens, query_lens, block_size, size, device) -> Optional[torch.Tensor]:
+def _slot_launches_suffice(context_lens, query_lens, block_size) -> bool:
+    """Whether sequences of these lengths fit ``_MAX_SLOT_LAUNCHES`` launches, each filled up in turn."""
+    if 4 * sum(map(bool, query_lens)) > _MAX_SLOT_LAUNCHES * (_lib.EMM_MAX_SLOT_WORDS - 1):
+        return False  # not even if every sequence had one block
+    launches = words = 1
+    for ctx, q in zip(context_lens, query_lens):
+        if type(ctx) is not int or type(q) is not int or ctx < 0 or q < 0:
+            return False
+        if q == 0:
+            continue
+        need = 4 + (ctx + q - 1) // block_size - ctx // block_size
+        words += need
+        if words > _lib.EMM_MAX_SLOT_WORDS:
+            launches, words = launches + 1, 1 + need
+            if launches > _MAX_SLOT_LAUNCHES or words > _lib.EMM_MAX_SLOT_WORDS:
+                return False
+    return True
+
+
+def _slot_mapping_on_device(block_tables, context_lens, query_lens, block_size, total, size, device) -> Optional[torch.Tensor]:
     """The slots written by a kernel from tables in its argument block; None for whatever does not fit
     ``_MAX_SLOT_LAUNCHES`` launches or is not a list of plain non-negative ids (the general path takes it)."""
+    # Tables that do not fit are found before anything is built from them. A sequence takes 3 words and one per block,
+    # of which its tokens touch at most q // block_size + 2 (a single token one): upper bounds on the words settle the
+    # usual step, an exact count is made only where they do not.
+    n, room = len(query_lens), _lib.EMM_MAX_SLOT_WORDS - 5  # what a launch surely holds, less the longest sequence's blocks
+    if 5 * n + total // block_size > _MAX_SLOT_LAUNCHES * (room - total // block_size):
+        ones = list(query_lens).count(1)
+        most = 4 * ones + 5 * (n - ones) + (total - ones) // block_size
+        if most > _MAX_SLOT_LAUNCHES * (room - max(query_lens) // block_size) and \
+                not _slot_launches_suffice(context_lens, query_lens, block_size):
+            return None
     launches = []
     starts, offsets, firsts, blocks = [0], [], [], []
     pos = 0
@@ -202,8 +231,6 @@ def _slot_mapping_on_device(block_tables, context_lens, query_lens, block_size, 
         if hi > len(table):
             return None
         if 3 * len(starts) + 1 + len(blocks) + hi - lo > _lib.EMM_MAX_SLOT_WORDS:
-            if 4 + hi - lo > _lib.EMM_MAX_SLOT_WORDS or len(launches) + 2 > _MAX_SLOT_LAUNCHES:
-                return None
             launches.append((starts, offsets, firsts, blocks))
             starts, offsets, firsts, blocks = [pos], [], [], []
         offsets.append(ctx - lo * block_size)
@@ -255,7 +282,7 @@ def compute_slot_mapping(block_tables: Sequence[Sequence[int]], context_lens: Se
         raise ValueError(f"pad_to={pad_to} is smaller than the {total} tokens of the step")
     gpu = device is not None and torch.device(device).type == "cuda"
     if gpu and 0 < size <= 0x7fffffff and type(block_size) is int and 0 < block_size <= 0x7fffffff:
-        on_device = _slot_mapping_on_device(block_tables, context_lens, query_lens, block_size, size, device)
+        on_device = _slot_mapping_on_device(block_tables, context_lens, query_lens, block_size, total, size, device)
         if on_device is not None:
             return on_device
     out = torch.empty(size, dtype=torch.long, pin_memory=gpu)

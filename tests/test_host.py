@@ -758,3 +758,57 @@ def test_every_operator_is_launched_on_its_tensors_gpu(monkeypatch):
     rig.launched_on_1("emm_concat_rows")
     kv_ops.stream_copy(key, new(T, H, D))
     rig.launched_on_1("emm_stream_copy")
+
+
+def test_slot_tables_that_do_not_fit_are_not_tried(monkeypatch):
+    """Tables beyond the launches' words go to the general path before anything is built from them; what fits is found
+    to fit, at every size around the limit."""
+    rig = OtherGpuIsCurrent(monkeypatch)
+    words, most = _lib.EMM_MAX_SLOT_WORDS, cache_ops._MAX_SLOT_LAUNCHES
+
+    class Tables(list):
+        passes = 0
+
+        def __iter__(self):
+            self.passes += 1
+            return super().__iter__()
+
+    def on_device(contexts, lengths, bs):
+        tables = Tables([list(range((c + q + bs - 1) // bs)) for c, q in zip(contexts, lengths)])
+        total = sum(lengths)
+        out = cache_ops._slot_mapping_on_device(tables, contexts, lengths, bs, total, total, "cuda:1")
+        launches, rig.calls = len(rig.calls), []
+        assert launches == 0 if out is None else 1 <= launches <= most
+        return out is not None, tables.passes
+
+    def fits(contexts, lengths, bs):  # filled up in turn: 3 words a sequence, one a block, one to close a launch
+        launches = used = 1
+        for c, q in zip(contexts, lengths):
+            if q == 0:
+                continue
+            need = 3 + (c + q - 1) // bs + 1 - c // bs
+            if need + 1 > words:
+                return False
+            if used + need > words:
+                launches, used = launches + 1, 1
+            used += need
+        return launches <= most
+
+    rng = np.random.default_rng(0)
+    cases = [([0] * n, [1] * n, 16) for n in (1, 239, 240, 955, 956, 957, 1500)]
+    cases += [([c], [16 * b], 16) for b in (955, 956, 957, 5000) for c in (0, 3)]
+    cases += [([5] * 1300 + [0], [1] * 1300 + [16 * 2000], 16), ([7] * 300 + [0], [1] * 300 + [8192], 16), ([0, 0], [0, 1], 16)]
+    for _ in range(300):
+        n, bs = int(rng.integers(1, 1200)), int(rng.choice([1, 3, 16, 128]))
+        top = int(rng.choice([1, 2, 17, 40, 400]))
+        cases.append((rng.integers(0, 300, n).tolist(), rng.integers(0, top + 1, n).tolist(), bs))
+    seen = set()
+    for contexts, lengths, bs in cases:
+        if sum(lengths) == 0:
+            continue
+        got, passes = on_device(contexts, lengths, bs)
+        want = fits(contexts, lengths, bs)
+        assert got == want, (len(lengths), bs, sum(lengths))
+        assert passes == (1 if want else 0), "tables that do not fit were walked"
+        seen.add(want)
+    assert seen == {True, False}
