@@ -1304,6 +1304,48 @@ def test_paged_append_every_dispatched_wave_shape(cache, H, D, bs, T, phase):
     assert same_bits(kc_g, kc) and same_bits(vc_g, vc)
 
 
+# per layer, 16-bit caches: single tokens written through below 64 pieces, both non-temporal from 2^30 tokens x elements^2
+@pytest.mark.parametrize("cache,H,D,bs,T,phase", [("auto", 5, 104, 16, 192, 3), ("auto", 5, 104, 16, 193, 0), ("auto", 5, 104, 16, 3970, 5),
+                                                  ("auto", 5, 104, 16, 3971, 9), ("auto", 9, 120, 32, 920, 1), ("auto", 9, 120, 32, 921, 14)])
+def test_paged_append_on_both_sides_of_its_store_policies(cache, H, D, bs, T, phase):
+    test_paged_append_every_dispatched_wave_shape(cache, H, D, bs, T, phase)
+
+
+# all layers in one launch: pieces = ceil(T / 16) * ceil(H * D / 128), weight = T * (H * D)^2. 16-bit: written through below
+# 448 pieces or 3 * 2^28, both non-temporal from 1152 pieces; fp8: the general kernel below 256 pieces
+@pytest.mark.parametrize("cache,H,D,bs,T,phase", [
+    ("auto", 5, 104, 16, 1424, 3), ("auto", 5, 104, 16, 2978, 0), ("auto", 5, 104, 16, 2979, 7), ("auto", 5, 104, 32, 3680, 1),
+    ("auto", 5, 104, 16, 3681, 11), ("auto", 9, 120, 16, 784, 2), ("auto", 9, 120, 64, 785, 5), ("auto", 2, 40, 16, 33, 6),
+    ("fp8", 5, 112, 16, 816, 3), ("fp8", 5, 112, 16, 817, 0), ("fp8_sat", 5, 112, 32, 816, 5), ("fp8_sat", 5, 112, 16, 817, 9),
+    ("fp8", 1, 16, 16, 5000, 1), ("fp8_sat", 4, 128, 16, 2561, 13)])
+def test_paged_append_all_layers_on_both_sides_of_its_rules(cache, H, D, bs, T, phase):
+    """Pointers, scales and shapes of every layer; sources are views of a wider projection, scales differ per layer."""
+    L, NB = 3, T // 6 + 60
+    dtype = torch.float16 if T % 2 else torch.bfloat16
+    say(f"paged append, all layers: {cache} H={H} D={D} bs={bs} T={T} phase={phase} {dtype}")
+    g = torch.Generator().manual_seed(T + H)
+    slots = paged_slots(NB, bs, T, seed=T + 1, phase=phase, pad_frac=0.01)
+    assert len(slots) == T
+    wide = (torch.randn((L, T, 2 * H * D), generator=g) * 40).to(dtype)
+    wide_g = wide.to(DEV)
+    keys, values, keys_g, values_g = ([w[l, :, i * H * D:(i + 1) * H * D].view(T, H, D) for l in range(L)]
+                                      for w in (wide, wide_g) for i in range(2))
+    ks, vs = torch.linspace(0.03, 0.09, L), torch.linspace(0.4, 0.2, L)  # part of the quotients overflow
+    caches = [paged_caches_cpu(NB, H, D, bs, dtype if cache == "auto" else torch.uint8, fill_mod=31 + l) for l in range(L)]
+    kcs, vcs = ([c[i].to(DEV) for c in caches] for i in range(2))
+    cache_ops.paged_layered_append(keys_g, values_g, kcs, vcs, cache, ks, vs)(slots.to(DEV))
+    for l, (kc, vc) in enumerate(caches):
+        k, v = keys[l].contiguous(), values[l].contiguous()
+        if cache == "auto":
+            orc.c_reshape_and_cache_paged(k, v, kc, vc, slots)
+        elif cache == "fp8":
+            orc.c_reshape_and_cache_paged(k, v, kc, vc, slots, float(ks[l]), float(vs[l]))
+        else:  # the bytes of the saturating cast, placed by the byte-copying reference
+            k8, v8 = (torch.from_numpy(orc.c_quant_fp8_sat(x, float(sc[l])).reshape(T, H, D).copy()) for x, sc in ((k, ks), (v, vs)))
+            orc.ref_reshape_and_cache_paged(k8, v8, kc, vc, slots)
+        assert same_bits(kcs[l], kc) and same_bits(vcs[l], vc), f"layer {l}"
+
+
 @pytest.mark.parametrize("bs,seqs,chunk,pad", [(16, 1, 0, 0), (16, 24, 0, 3), (16, 239, 0, 0), (16, 240, 0, 0), (12, 400, 1000, 7),
                                                (16, 0, 16 * 956, 0), (16, 0, 16 * 956 + 1, 5), (16, 30, 8192, 300), (1, 5, 700, 0),
                                                (16, 1200, 40, 0), (256, 3, 5000, 1)])
