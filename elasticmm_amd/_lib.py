@@ -6,9 +6,9 @@ the caller gets an exception.
 from __future__ import annotations
 
 import ctypes
+import functools
 import importlib.util
 import os
-import sys
 from ctypes import c_char_p, c_float, c_int, c_int64, c_void_p, POINTER
 
 from .build import frontend_path, hooks_library_path, library_path
@@ -86,24 +86,35 @@ class EmmError(RuntimeError):
 _frontend_module = None
 
 
-def _bind_frontend(lib: ctypes.CDLL) -> None:
-    """``lib.frontend``: the native host side of the per-layer appends (csrc/emm_frontend.cpp) over this library's
-    entry points. Without torch there are no tensors to check and only the C ABI is bound."""
+def _load_frontend():
+    """The extension module of csrc/emm_frontend.cpp, built for this Python and this torch."""
     global _frontend_module
-    if "torch" not in sys.modules:
-        return
     if _frontend_module is None:
+        import torch
+
         path = frontend_path()
         if not os.path.exists(path):
-            raise RuntimeError(f"{path} is missing: the native host side has not been built "
+            raise RuntimeError(f"{path} is missing: the native host side of the appends has not been built for this Python "
                                "(run `python -m elasticmm_amd.build`)")
         spec = importlib.util.spec_from_file_location("_emm_frontend", path)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
+        if module.TORCH_VERSION != torch.__version__.split("+")[0]:
+            raise RuntimeError(f"{path} was built for torch {module.TORCH_VERSION}, this is {torch.__version__} "
+                               "(run `python -m elasticmm_amd.build`)")
         _frontend_module = module
-    address = lambda fn: ctypes.cast(fn, c_void_p).value  # noqa: E731
-    lib.frontend = _frontend_module.Frontend(address(lib.emm_reshape_and_cache), address(lib.emm_reshape_and_cache_fp8),
-                                             address(lib.emm_reshape_and_cache_paged))
+    return _frontend_module
+
+
+class Library(ctypes.CDLL):
+    """One of the two shared objects, with the native host side of the per-layer appends over its entry points."""
+
+    @functools.cached_property
+    def frontend(self):
+        """Loaded by the first append that asks for it: nothing else needs it, nor torch's headers to be built."""
+        address = lambda fn: ctypes.cast(fn, c_void_p).value  # noqa: E731
+        return _load_frontend().Frontend(self.emm_abi_version(), address(self.emm_reshape_and_cache),
+                                         address(self.emm_reshape_and_cache_fp8), address(self.emm_reshape_and_cache_paged))
 
 
 def load() -> ctypes.CDLL:
@@ -122,7 +133,7 @@ def load() -> ctypes.CDLL:
         import torch  # noqa: F401
     except ImportError:
         pass
-    lib = ctypes.CDLL(path)
+    lib = Library(path)
     for name, (res, args) in SIGNATURES.items():
         fn = getattr(lib, name)  # AttributeError if the symbol is not exported
         fn.restype = res
@@ -130,7 +141,6 @@ def load() -> ctypes.CDLL:
     ver = lib.emm_abi_version()
     if ver != EMM_KV_ABI_VERSION:
         raise RuntimeError(f"libemm_kv.so ABI version {ver}, expected {EMM_KV_ABI_VERSION}")
-    _bind_frontend(lib)
     _lib = lib
     return lib
 
@@ -147,12 +157,11 @@ def load_hooks() -> ctypes.CDLL:
         import torch  # noqa: F401
     except ImportError:
         pass
-    lib = ctypes.CDLL(path)
+    lib = Library(path)
     for name, (res, args) in {**SIGNATURES, **HOOK_SIGNATURES}.items():
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
-    _bind_frontend(lib)
     _hooks = lib
     return lib
 

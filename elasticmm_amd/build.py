@@ -1,10 +1,12 @@
-"""In-tree build of libemm_kv.so with hipcc for gfx950, and of the native host side of the appends (_emm_frontend.so).
+"""In-tree build of libemm_kv.so with hipcc for gfx950, and of the native host side of the
+appends (_emm_frontend, an extension module of the Python and the torch it is built with).
 
 The shared object is written next to this file so that it travels with the
 source tree; nothing is installed and no JIT cache is used.
 """
 from __future__ import annotations
 
+import importlib.util
 import os
 import shutil
 import subprocess
@@ -16,7 +18,7 @@ _SRC = os.path.join(_PKG, "csrc", "emm_kv.hip")
 _INC = os.path.join(_ROOT, "include")
 _OUT = os.path.join(_PKG, "libemm_kv.so")
 _SRC_FRONTEND = os.path.join(_PKG, "csrc", "emm_frontend.cpp")
-_OUT_FRONTEND = os.path.join(_PKG, "_emm_frontend.so")
+_OUT_FRONTEND = os.path.join(_PKG, "_emm_frontend" + sysconfig.get_config_var("EXT_SUFFIX"))
 _OUT_HOOKS = os.path.join(_PKG, "libemm_kv_hooks.so")
 
 HIPCC_FLAGS = [
@@ -49,7 +51,7 @@ def frontend_path() -> str:
 
 
 def build_frontend(verbose: bool = False) -> str:
-    """Compile csrc/emm_frontend.cpp -> _emm_frontend.so against the installed torch (always recompiles)."""
+    """Compile csrc/emm_frontend.cpp -> _emm_frontend.<python tag>.so against the installed torch (always recompiles)."""
     import torch
 
     root = os.path.dirname(torch.__file__)
@@ -75,8 +77,8 @@ def build_library(verbose: bool = False, hooks: bool = False) -> str:
     libemm_kv_hooks.so instead: the same source with -DEMM_BENCH_HOOKS, which adds the launch-variant
     switch, the memory-system probes and the quotient sweep that bench.py and the GPU tests use
     (csrc/emm_kv_hooks.h, csrc/emm_kv_hooks.inc). The product library never contains them; with it the native host
-    side of the appends (``build_frontend``) is built."""
-    if not hooks:
+    side of the appends (``build_frontend``) is built where torch is installed."""
+    if not hooks and importlib.util.find_spec("torch") is not None:
         build_frontend(verbose)
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     out = _OUT_HOOKS if hooks else _OUT

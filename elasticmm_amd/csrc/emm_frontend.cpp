@@ -17,6 +17,7 @@
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/headeronly/version.h>
 
 #include "emm_kv.h"
 
@@ -171,8 +172,12 @@ PyMethodDef frontend_methods[] = {
     {nullptr, nullptr, 0, nullptr}};
 
 PyObject *frontend_new(PyTypeObject *type, PyObject *args, PyObject *) {
+  int version; // of the library the entry points belong to: their signatures are those of this file's emm_kv.h or others
   unsigned long long a, b, c; // addresses of the three entry points
-  if (!PyArg_ParseTuple(args, "KKK", &a, &b, &c)) return nullptr;
+  if (!PyArg_ParseTuple(args, "iKKK", &version, &a, &b, &c)) return nullptr;
+  if (version != EMM_KV_ABI_VERSION)
+    return PyErr_Format(PyExc_RuntimeError, "the native host side was built for ABI version %d, the library has %d", EMM_KV_ABI_VERSION, version);
+  if (!a || !b || !c) return PyErr_Format(PyExc_ValueError, "null entry point");
   Frontend *f = reinterpret_cast<Frontend *>(type->tp_alloc(type, 0));
   if (!f) return nullptr;
   f->append = reinterpret_cast<append_fn>(a);
@@ -195,6 +200,10 @@ PyMODINIT_FUNC PyInit__emm_frontend(void) {
   if (PyType_Ready(&frontend_type) < 0) return nullptr;
   PyObject *m = PyModule_Create(&module_def);
   if (!m) return nullptr;
+  if (PyModule_AddStringConstant(m, "TORCH_VERSION", TORCH_VERSION) < 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
   Py_INCREF(&frontend_type);
   if (PyModule_AddObject(m, "Frontend", reinterpret_cast<PyObject *>(&frontend_type)) < 0) {
     Py_DECREF(&frontend_type);

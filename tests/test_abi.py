@@ -181,3 +181,35 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "library_path", lambda: str(tmp_path / "nope.so"))
     with pytest.raises(RuntimeError, match="no CPU fallback"):
         _lib.load()
+
+
+def test_native_host_side_is_loaded_by_the_appends_only(monkeypatch, tmp_path):
+    """pack, unpack and migrate work without the extension module; an append asks for it and says what is missing."""
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "_frontend_module", None)
+    monkeypatch.setattr(_lib, "frontend_path", lambda: str(tmp_path / "nope.so"))
+    lib = _lib.load()
+    assert lib.emm_kv_pack(_lib.ptr_table([0x1000]), 1, 2, 4, 64, None, 0, None, None) == 0
+    with pytest.raises(RuntimeError, match="native host side"):
+        lib.frontend
+    monkeypatch.undo()
+    assert _lib.load().frontend is _lib.load().frontend
+
+
+def test_native_host_side_of_another_build_is_refused(monkeypatch):
+    """An extension compiled against another header would call the entry points with other signatures; one compiled
+    against another torch would read other tensors."""
+    module = _lib._load_frontend()
+    for version in (0, _lib.EMM_KV_ABI_VERSION - 1, _lib.EMM_KV_ABI_VERSION + 1):
+        with pytest.raises(RuntimeError, match="ABI version"):
+            module.Frontend(version, 0x1000, 0x1000, 0x1000)
+    with pytest.raises(ValueError, match="null entry point"):
+        module.Frontend(_lib.EMM_KV_ABI_VERSION, 0x1000, 0, 0x1000)
+    with pytest.raises(TypeError):
+        module.Frontend(0x1000, 0x1000, 0x1000)
+    import torch
+
+    monkeypatch.setattr(_lib, "_frontend_module", None)
+    monkeypatch.setattr(torch, "__version__", "1.0.0+rocm0")
+    with pytest.raises(RuntimeError, match="built for torch"):
+        _lib._load_frontend()
