@@ -66,7 +66,12 @@ bool take(PyObject *const *args, Py_ssize_t nargs, Call &c, int &mode) {
   if (!(c.key = usual(args[0])) || !(c.value = usual(args[1])) || !(c.kc = usual(args[2])) ||
       !(c.vc = usual(args[3])) || !(c.slots = usual(args[4])))
     return false;
-  mode = (int)PyLong_AsLong(args[5]);
+  const long m = PyLong_AsLong(args[5]);
+  if (m == -1 && PyErr_Occurred()) { // not a number: the Python operator says so
+    PyErr_Clear();
+    return false;
+  }
+  mode = (int)m;
   const at::Device device = c.key->device();
   if (c.value->device() != device || c.kc->device() != device || c.vc->device() != device || c.slots->device() != device)
     return false;

@@ -1441,24 +1441,35 @@ def test_native_append_takes_the_usual_calls_only(layout, cache):
     class Sub(torch.Tensor):
         pass
 
-    odd = [(key.as_subclass(Sub), value, slots, one), (key, value, slots.repeat_interleave(2)[::2], one),
-           (key.permute(2, 1, 0).contiguous().permute(2, 1, 0), value, slots, one), (key, value, slots.int(), one),
-           (key, value, slots[:-1], one), (key[:0], value[:0], slots, one), (key, value[:, :1], slots, one),
-           (key, value, slots.cpu(), one)]
+    # (call, what the operator makes of it: the usual bytes, nothing at all, or an error)
+    same, nothing = "same", "nothing"
+    odd = [(key.as_subclass(Sub), value, slots, one, same), (key, value, slots.repeat_interleave(2)[::2], one, same),
+           (key.permute(2, 1, 0).contiguous().permute(2, 1, 0), value, slots, one, ValueError), (key, value, slots.int(), one, TypeError),
+           (key, value, slots[:-1], one, ValueError), (key[:0], value[:0], slots, one, nothing),
+           (key, value[:, :1], slots, one, ValueError),
+           (key, value, slots.cpu(), one, RuntimeError if layout == "flash" else TypeError)]
     if layout == "flash":
-        odd.append((key.view(T, H * D), value.view(T, H * D), slots, one))
+        odd.append((key.view(T, H * D), value.view(T, H * D), slots, one, same))
     if cache != "auto":
-        odd += [(key, value, slots, one.double()), (key, value, slots, None), (key, value, slots, 0.05), (key.float(), value.float(), slots, one)]
-    for n, (k, v, s, sc) in enumerate(odd):
+        odd += [(key, value, slots, one.double(), same), (key, value, slots, None, ValueError), (key, value, slots, 0.05, same),
+                (key.float(), value.float(), slots, one, TypeError)]
+    for n, (k, v, s, sc, outcome) in enumerate(odd):
         c = caches()
         assert native(k, v, *c, s, mode, sc, sc) == 0, f"odd call {n}"
         assert all(bool((t == 7).all()) for t in c), f"odd call {n} wrote"
-        try:
+        if outcome in (same, nothing):
             op(k, v, *c, s, cache, sc, sc)
-        except (ValueError, TypeError, RuntimeError):
-            continue
-        if k.numel():
-            assert same_bits(c[0], want[0]) and same_bits(c[1], want[1]), f"odd call {n}"
+            if outcome == same:
+                assert same_bits(c[0], want[0]) and same_bits(c[1], want[1]), f"odd call {n}"
+                continue
+        else:
+            with pytest.raises(outcome):
+                op(k, v, *c, s, cache, sc, sc)
+        assert all(bool((t == 7).all()) for t in c), f"odd call {n} wrote"
+    c = caches()
+    for not_a_mode in ("auto", None, 2 ** 70, -1, 3):
+        assert native(key, value, *c, slots, not_a_mode, one, one) == 0
+    assert all(bool((t == 7).all()) for t in c)
 
 
 @pytest.mark.skipif(torch.cuda.device_count() < 2, reason="needs a second GPU")
