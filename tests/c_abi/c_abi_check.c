@@ -2,7 +2,7 @@
  * A C program (no Python, no torch) that drives libemm_kv.so through include/emm_kv.h and checks
  * every data-moving entry point (pack, unpack, their host-table forms, copy_blocks, migrate, the appends in the
  * flash, strided and paged layouts, 16-bit and fp8, per layer and for all layers, the dequantising unpack,
- * concat_rows, the plain copy) against the loops of oracle/kv_oracle.c on seeded data. Built and run by tests/test_c_abi_program.py.
+ * the slot mapping, concat_rows, the plain copy) against the loops of oracle/kv_oracle.c on seeded data. Built and run by tests/test_c_abi_program.py.
  *
  *   gcc -std=c11 -O2 -D__HIP_PLATFORM_AMD__ -Iinclude -I/opt/rocm/include -o tests/c_abi/c_abi_check \
  *       tests/c_abi/c_abi_check.c oracle/kv_oracle.c -Lelasticmm_amd -lemm_kv -L/opt/rocm/lib -lamdhip64 -lm \
@@ -244,6 +244,36 @@ int main(void) {
   orc_kv_unpack(h_dst, L, KV, NB, chunk, h_di3, N, h_want);
   for (int l = 0; l < L; ++l) bad += same_on_device(d_dst[l], h_dst[l], layer_bytes, "emm_kv_migrate");
 
+  /* the same with both tables on the host; two pairs reach outside a pool and are skipped */
+  permutation(h_si3, NB, N);
+  permutation(h_di3, NB, N);
+  h_si3[2] = -1;
+  h_di3[5] = NB;
+  EMM(emm_kv_migrate_host_ids((const void *const *)d_src, NB, d_dst, NB, L, KV, chunk, h_si3, h_di3, N, stream));
+  int64_t h_si4[N], h_di4[N], n4 = 0;
+  for (int i = 0; i < N; ++i)
+    if (i != 2 && i != 5) h_si4[n4] = h_si3[i], h_di4[n4++] = h_di3[i];
+  orc_kv_pack((const void *const *)h_src, L, KV, NB, chunk, h_si4, n4, h_want);
+  orc_kv_unpack(h_dst, L, KV, NB, chunk, h_di4, n4, h_want);
+  for (int l = 0; l < L; ++l) bad += same_on_device(d_dst[l], h_dst[l], layer_bytes, "emm_kv_migrate_host_ids");
+
+  /* the slots of a step: a decode token, a prompt over three blocks, a chunk that starts inside its block, two padded */
+  {
+    const int64_t starts[4] = {0, 1, 41, 50}, offsets[3] = {11, 0, 5}, firsts[3] = {0, 1, 4}, ids[5] = {7, 30, 2, 2147483647, 19};
+    int64_t want[52];
+    for (int i = 0; i < 3; ++i)
+      for (int64_t t = starts[i]; t < starts[i + 1]; ++t) {
+        const int64_t p = offsets[i] + t - starts[i];
+        want[t] = ids[firsts[i] + p / 16] * 16 + p % 16;
+      }
+    want[50] = want[51] = -1;
+    memset(h_want, 0x55, sizeof(want) + 8);
+    int64_t *d_out = (int64_t *)to_device(h_want, sizeof(want) + 8);
+    memcpy(h_want, want, sizeof(want)); /* the word behind the output stays as it was */
+    EMM(emm_slot_mapping(starts, offsets, firsts, 3, ids, 5, 16, 52, d_out, stream));
+    bad += same_on_device(d_out, h_want, sizeof(want) + 8, "emm_slot_mapping");
+  }
+
   /* the append for all layers in one launch, token rows 8 bytes further apart than they are long */
   enum { BS = 16, H = 2, D = 64 };
   const int64_t row_elems = H * D, stride_elems = row_elems + 4;
@@ -366,6 +396,13 @@ int main(void) {
     EMM(emm_kv_unpack_dequant_fp8(d_dst, L, NB, chunk_elems, d_di, N, d_packed8, d_ks, d_vs, EMM_DTYPE_BF16, stream));
     orc_kv_unpack_dequant_fp8(h_dst, L, NB, chunk_elems, h_di, N, h_packed8, h_ks, h_vs, EMM_DTYPE_BF16);
     for (int l = 0; l < L; ++l) bad += same_on_device(d_dst[l], h_dst[l], layer_bytes, "emm_kv_unpack_dequant_fp8");
+    int64_t h_di5[N];
+    permutation(h_di5, NB, N);
+    h_di5[1] = -1; /* skipped */
+    h_di5[4] = NB;
+    EMM(emm_kv_unpack_dequant_fp8_host_ids(d_dst, L, NB, chunk_elems, h_di5, N, d_packed8, d_ks, d_vs, EMM_DTYPE_F16, stream));
+    orc_kv_unpack_dequant_fp8(h_dst, L, NB, chunk_elems, h_di5, N, h_packed8, h_ks, h_vs, EMM_DTYPE_F16);
+    for (int l = 0; l < L; ++l) bad += same_on_device(d_dst[l], h_dst[l], layer_bytes, "emm_kv_unpack_dequant_fp8_host_ids");
 
     /* paged-attention layout: one prompt filling blocks in order plus scattered tokens; 16-bit and fp8 caches */
     enum { TP = 50 };

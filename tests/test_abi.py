@@ -61,6 +61,8 @@ def test_binding_table_matches_header():
     assert int(re.search(r"#define EMM_MAX_LAYERS (\d+)", text).group(1)) == _lib.EMM_MAX_LAYERS
     assert int(re.search(r"#define EMM_MAX_SEGMENTS (\d+)", text).group(1)) == _lib.EMM_MAX_SEGMENTS
     assert int(re.search(r"#define EMM_KV_ABI_VERSION (\d+)", text).group(1)) == _lib.EMM_KV_ABI_VERSION
+    for name in ("EMM_MAX_INLINE_IDS", "EMM_MAX_INLINE_PAIRS", "EMM_MAX_INLINE_PAIRS_TABLES", "EMM_MAX_SLOT_WORDS"):
+        assert int(re.search(rf"#define {name} (\d+)", text).group(1)) == getattr(_lib, name)
 
 
 def test_load_and_argument_errors_without_gpu():
@@ -110,6 +112,30 @@ def test_argument_errors_of_the_layout_variants_without_gpu():
     rc = lib.emm_reshape_and_cache_strided(t, t, t, t, 1, P, 4, 2, 64, 16, 8, 100, 128, 4096, 128, 64, None)
     assert rc == -1 and b"token stride" in lib.emm_last_error()
     assert lib.emm_reshape_and_cache_strided(t, t, t, t, 0, P, 4, 2, 64, 16, 8, 128, 128, 4096, 128, 64, None) == 0
+
+
+def test_argument_errors_of_the_host_table_moves_without_gpu():
+    lib = _lib.load()
+    P, t, none = 0x1000, _lib.ptr_table([0x1000]), _lib.ptr_table([0])
+
+    def migrate(src=t, src_nb=4, dst=t, dst_nb=4, layers=1, kv=2, chunk=64, si=P, di=P, n=1):
+        return lib.emm_kv_migrate_host_ids(src, src_nb, dst, dst_nb, layers, kv, chunk, si, di, n, None)
+
+    def dequant(table=t, layers=1, nb=4, chunk=32, ids=P, n=1, packed=P, ks=P, vs=P, dtype=0):
+        return lib.emm_kv_unpack_dequant_fp8_host_ids(table, layers, nb, chunk, ids, n, packed, ks, vs, dtype, None)
+
+    for call, text, kw in [(migrate, b"num_layers", {"layers": 97}), (migrate, b"negative", {"chunk": -1}), (migrate, b"negative", {"dst_nb": -1}),
+                           (migrate, b"negative", {"n": -1}), (migrate, b"exceeds", {"src_nb": 2 ** 31}), (migrate, b"exceeds", {"dst_nb": 2 ** 31}),
+                           (migrate, b"null", {"src": None}), (migrate, b"null", {"dst": none}), (migrate, b"null index", {"si": None}),
+                           (migrate, b"null index", {"di": None}),
+                           (dequant, b"num_layers", {"layers": 97}), (dequant, b"negative", {"nb": -1}), (dequant, b"out_dtype", {"dtype": 2}),
+                           (dequant, b"null", {"ids": None}), (dequant, b"null", {"packed": None}), (dequant, b"null", {"ks": None}),
+                           (dequant, b"null", {"vs": None}), (dequant, b"multiples of 16", {"chunk": 24}),
+                           (dequant, b"multiples of 16", {"packed": P + 8}), (dequant, b"aligned", {"table": _lib.ptr_table([P + 8])}),
+                           (dequant, b"too large", {"chunk": 2 ** 31})]:
+        assert call(**kw) == -1 and text in lib.emm_last_error() and b"host_ids" in lib.emm_last_error(), (kw, lib.emm_last_error())
+    for empty in ({"n": 0}, {"layers": 0}, {"chunk": 0}):
+        assert migrate(si=None, di=None, **empty) == 0 and dequant(ids=None, packed=None, **empty) == 0
 
 
 def test_argument_errors_of_the_slot_mapping_without_gpu():

@@ -1740,6 +1740,39 @@ def test_host_id_entry_points_match_the_device_table_ones():
 
 
 
+@pytest.mark.parametrize("equal", [True, False], ids=["equally spaced planes", "separate layers"])
+def test_host_table_moves_skip_ids_out_of_range(equal):
+    """The C ABI directly: a pair, or an id, outside its pool is skipped and every other block of the pool stays as it is."""
+    lib = _lib.load()
+    L, NBs, NBd = 2, 40, 24
+    src_c, dst_c = cpu_pool(L, NBs, 16, 2, 64, torch.bfloat16, 3), cpu_pool(L, NBd, 16, 2, 64, torch.bfloat16, 0, fill=-1.0)
+    src, dst = (PoolView(to_dev(p, equal)) for p in (src_c, dst_c))
+    stream = torch.cuda.current_stream().cuda_stream
+    si = np.array([3, -1, 39, 40, 7, 5, 10 ** 12, 6], dtype=np.int64)
+    di = np.array([1, 2, 23, 3, -1, 24, 4, 0], dtype=np.int64)
+    rc = lib.emm_kv_migrate_host_ids(_lib.ptr_table(src.ptrs), NBs, _lib.ptr_table(dst.ptrs), NBd, L, 2, src.chunk_bytes,
+                                     si.ctypes.data, di.ctypes.data, len(si), stream)
+    assert rc == 0, lib.emm_last_error()
+    for l in range(L):
+        for a, b in zip(si.tolist(), di.tolist()):
+            if 0 <= a < NBs and 0 <= b < NBd:
+                dst_c[l][:, b] = src_c[l][:, a]
+        assert same_bits(dst.layers[l], dst_c[l]) and same_bits(src.layers[l], src_c[l]), f"migrate, layer {l}"
+    ids = np.array([5, -1, 23, 24, 2 ** 32, 0], dtype=np.int64)
+    packed = torch.randint(0, 0x7F, (L, 2, len(ids), 16, 2, 64), dtype=torch.uint8, generator=torch.Generator().manual_seed(4))
+    ks, vs = torch.tensor([0.02, 0.3]), torch.tensor([0.5, 0.07])
+    packed_g, ks_g, vs_g = packed.to(DEV), ks.to(DEV), vs.to(DEV)
+    rc = lib.emm_kv_unpack_dequant_fp8_host_ids(_lib.ptr_table(dst.ptrs), L, NBd, dst.chunk_elems, ids.ctypes.data, len(ids),
+                                                packed_g.data_ptr(), ks_g.data_ptr(), vs_g.data_ptr(), 0, stream)
+    assert rc == 0, lib.emm_last_error()
+    values = packed.view(torch.float8_e4m3fn).float() * torch.stack([ks, vs], 1).view(L, 2, 1, 1, 1, 1)
+    for l in range(L):
+        for j, b in enumerate(ids.tolist()):
+            if 0 <= b < NBd:
+                dst_c[l][:, b] = values[l, :, j].to(torch.bfloat16)
+        assert same_bits(dst.layers[l], dst_c[l]), f"dequantising unpack, layer {l}"
+
+
 # ------------------------------------------------------------------ worker protocol
 def make_pair(L=3, NB=32, bs=16, H=2, D=64, dtype=torch.bfloat16):
     link = LoopbackLink(world_size=2)
