@@ -248,16 +248,17 @@ def _slot_mapping_on_device(block_tables, context_lens, query_lens, block_size, 
         if ids and (min(ids) < 0 or max(ids) > 0x7fffffff):
             return None
     out = torch.empty(size, dtype=torch.long, device=device)
-    if kv_ops._elsewhere(out.device):
-        with torch.cuda.device(out.device):
-            _write_slots(packed, block_size, out)
-    else:
-        _write_slots(packed, block_size, out)
+    gpu, here = out.get_device(), kv_ops._get_device()
+    if gpu == here:
+        _write_slots(packed, block_size, out, gpu)
+    else:  # the launch goes to the current GPU, whatever the stream
+        with torch.cuda.device(gpu):
+            _write_slots(packed, block_size, out, gpu)
     return out
 
 
-def _write_slots(packed, block_size: int, out: torch.Tensor) -> None:
-    lib, stream, ptr, size = _lib.load(), kv_ops._stream_ptr(out.device), out.data_ptr(), out.numel()
+def _write_slots(packed, block_size: int, out: torch.Tensor, gpu: int) -> None:
+    lib, stream, ptr, size = _lib.load(), kv_ops._raw_stream(gpu), out.data_ptr(), out.numel()
     for n, (s, o, f, b) in enumerate(packed):
         _lib.check(lib.emm_slot_mapping(s.buffer_info()[0], o.buffer_info()[0], f.buffer_info()[0], len(o), b.buffer_info()[0],
                                         len(b), block_size, size if n == len(packed) - 1 else s[-1], ptr, stream), "emm_slot_mapping")

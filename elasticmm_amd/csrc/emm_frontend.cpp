@@ -97,9 +97,10 @@ bool take(PyObject *const *args, Py_ssize_t nargs, Call &c, int &mode) {
 }
 
 // The launch goes to the current device whatever the stream (the default stream's handle is null on every device):
-// the tensors' device has to be current.
+// the tensors' device has to be current. Asking which one is costs 0.1 us of a call's 3; where only one GPU is visible,
+// it is the one.
 void make_current(const Call &c, c10::OptionalDeviceGuard &guard) {
-  if (c10::hip::current_device() != c.key->device().index()) guard.reset_device(c.key->device());
+  if (c10::hip::device_count() > 1 && c10::hip::current_device() != c.key->device().index()) guard.reset_device(c.key->device());
 }
 
 PyObject *not_usual() { return PyLong_FromLong(0); }

@@ -663,7 +663,7 @@ class OtherGpuIsCurrent:
 
         class Device:
             def __init__(self, device):
-                self.index = torch.device(device).index
+                self.index = device if type(device) is int else torch.device(device).index
 
             def __enter__(self):
                 self.back, rig.current = rig.current, self.index
@@ -700,6 +700,9 @@ class OnGpu1:
 
     def __init__(self, t):
         self._t = t
+
+    def get_device(self):
+        return 1
 
     def __getattr__(self, name):
         return getattr(self._t, name)
