@@ -1304,21 +1304,20 @@ def test_paged_append_every_dispatched_wave_shape(cache, H, D, bs, T, phase):
     assert same_bits(kc_g, kc) and same_bits(vc_g, vc)
 
 
-# per layer, 16-bit caches: single tokens written through below 64 pieces, both non-temporal from 2^30 tokens x elements^2
+# per layer, 16-bit caches: single tokens written through up to 128 pieces
 # fp8: the general kernel up to 1024 pieces and from 1440 to 2048
 @pytest.mark.parametrize("cache,H,D,bs,T,phase", [("fp8", 20, 128, 16, 1136, 3), ("fp8_sat", 20, 128, 16, 1137, 0), ("fp8_sat", 20, 128, 16, 1632, 7),
-                                                  ("fp8", 20, 128, 32, 1633, 2), ("auto", 5, 104, 16, 192, 3), ("auto", 5, 104, 16, 193, 0), ("auto", 5, 104, 16, 3970, 5),
-                                                  ("auto", 5, 104, 16, 3971, 9), ("auto", 9, 120, 32, 920, 1), ("auto", 9, 120, 32, 921, 14)])
+                                                  ("fp8", 20, 128, 32, 1633, 2), ("auto", 5, 104, 16, 400, 3), ("auto", 5, 104, 16, 401, 0),
+                                                  ("auto", 9, 120, 32, 224, 1), ("auto", 9, 120, 32, 225, 14)])
 def test_paged_append_on_both_sides_of_its_rules(cache, H, D, bs, T, phase):
     test_paged_append_every_dispatched_wave_shape(cache, H, D, bs, T, phase)
 
 
-# all layers in one launch: pieces = ceil(T / 16) * ceil(H * D / 128), weight = T * (H * D)^2. 16-bit: written through below
-# 448 pieces or 3 * 2^28, both non-temporal from 1152 pieces; fp8: the general kernel below 256 pieces and, with rows of more
-# than 512 elements, from 640 pieces
+# all layers in one launch: pieces = ceil(T / 16) * ceil(H * D / 128). 16-bit: single tokens written through below 448 pieces,
+# non-temporal from there; fp8: the general kernel below 256 pieces and, with rows of more than 512 elements, from 640 pieces
 @pytest.mark.parametrize("cache,H,D,bs,T,phase", [
-    ("auto", 5, 104, 16, 1424, 3), ("auto", 5, 104, 16, 2978, 0), ("auto", 5, 104, 16, 2979, 7), ("auto", 5, 104, 32, 3680, 1),
-    ("auto", 5, 104, 16, 3681, 11), ("auto", 9, 120, 16, 784, 2), ("auto", 9, 120, 64, 785, 5), ("auto", 2, 40, 16, 33, 6),
+    ("auto", 5, 104, 16, 1424, 3), ("auto", 5, 104, 16, 1425, 0), ("auto", 5, 104, 32, 3680, 1), ("auto", 9, 120, 16, 784, 2),
+    ("auto", 9, 120, 64, 785, 5), ("auto", 2, 40, 16, 33, 6),
     ("fp8", 5, 112, 16, 816, 3), ("fp8", 5, 112, 16, 817, 0), ("fp8_sat", 5, 112, 32, 816, 5), ("fp8_sat", 5, 112, 16, 817, 9),
     ("fp8", 1, 16, 16, 5000, 1), ("fp8_sat", 4, 128, 16, 2561, 13), ("fp8", 5, 112, 16, 2032, 6), ("fp8_sat", 5, 112, 16, 2033, 2)])
 def test_paged_append_all_layers_on_both_sides_of_its_rules(cache, H, D, bs, T, phase):
