@@ -134,7 +134,9 @@ class PoolView:
                 raise ValueError(f"layer {i} is not contiguous")
         self.layers: List[torch.Tensor] = layers
         self.device = first.device if pinned_host_for is None else torch.device(pinned_host_for)
-        self.gpu = self.device.index  # None: whichever is current
+        # the GPU's index where a launch has to ask which one is current (``_elsewhere`` without its cost for a single GPU:
+        # pack and unpack run in front of kernels of a few microseconds)
+        self.one_of_several = self.device.index if torch.cuda.device_count() > 1 else None
         self.on_host = pinned_host_for is not None
         self.dtype = first.dtype
         self.elem_bytes = first.element_size()
@@ -216,8 +218,7 @@ def kv_pack(pool: PoolView, block_indices: IndexLike, out: Optional[torch.Tensor
     the allocation held. ``strict=True`` validates a device table first (``check_device_block_ids``: one
     reduction and a synchronisation) and raises ``IndexError`` instead."""
     lib = _lib.load()
-    here = _get_device()  # (_elsewhere, spelt out: this runs in front of kernels of a few microseconds)
-    if pool.gpu != here and pool.gpu is not None:
+    if pool.one_of_several is not None and pool.one_of_several != _get_device():
         with torch.cuda.device(pool.device):
             return kv_pack(pool, block_indices, out, strict)
     n, table_arg, inline, keep = _table_for_launch(block_indices, pool, strict, "kv_pack")
@@ -226,7 +227,7 @@ def kv_pack(pool: PoolView, block_indices: IndexLike, out: Optional[torch.Tensor
     elif out.device != pool.device or out.dtype != pool.dtype or not out.is_contiguous() \
             or out.numel() != pool.num_layers * pool.num_kv * n * pool.chunk_elems:
         raise ValueError("kv_pack: `out` must be a contiguous pool-dtype tensor of the packed size")
-    stream = _raw_stream(here)
+    stream = _stream_ptr(pool.device)
     plane = pool.num_kv * n * pool.chunk_bytes
     fn = lib.emm_kv_pack_host_ids if inline else lib.emm_kv_pack
     base = out.data_ptr()
@@ -244,8 +245,7 @@ def kv_unpack(pool: PoolView, block_indices: IndexLike, packed: torch.Tensor, st
     lib = _lib.load()
     if not packed.is_cuda:
         _require_gpu(packed, "kv_unpack")
-    here = _get_device()  # (_elsewhere, spelt out: this runs in front of kernels of a few microseconds)
-    if pool.gpu != here and pool.gpu is not None:
+    if pool.one_of_several is not None and pool.one_of_several != _get_device():
         with torch.cuda.device(pool.device):
             return kv_unpack(pool, block_indices, packed, strict)
     n, table_arg, inline, keep = _table_for_launch(block_indices, pool, strict, "kv_unpack")
@@ -257,7 +257,7 @@ def kv_unpack(pool: PoolView, block_indices: IndexLike, packed: torch.Tensor, st
                          f"pool geometry needs {pool.num_layers * pool.num_kv * n * pool.chunk_bytes}")
     if not packed.is_contiguous():
         packed = packed.contiguous()
-    stream = _raw_stream(here)
+    stream = _stream_ptr(pool.device)
     plane = pool.num_kv * n * pool.chunk_bytes
     fn = lib.emm_kv_unpack_host_ids if inline else lib.emm_kv_unpack
     base = packed.data_ptr()

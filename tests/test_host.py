@@ -681,6 +681,7 @@ class OtherGpuIsCurrent:
                 return entry
 
         monkeypatch.setattr(torch.cuda, "device", Device)
+        monkeypatch.setattr(torch.cuda, "device_count", lambda: 2)
         monkeypatch.setattr(kv_ops, "_get_device", lambda: rig.current)
         monkeypatch.setattr(kv_ops, "_raw_stream", lambda index: 0)
         monkeypatch.setattr(_lib, "_lib", Lib())
