@@ -19,7 +19,7 @@ extern "C" {
 /* Launch variants of the hooks library's own kernels: 0 = the product's defaults.
  * bits 8-11: 1 = non-temporal stores in the 16-byte block moves (default: sc0 sc1);
  * bits 12-15: shape of the 16-byte copy append (token rows per wave, waves per workgroup):
- *   0 = default ((4, 1) for a per-layer launch, (1, 1) for a whole-step launch), 1 = (1, 4), 2 = (2, 4),
+ *   0 = default (by token count and row length; (1, 1) for a whole-step launch), 1 = (1, 4), 2 = (2, 4),
  *   3 = (4, 1), 4 = (1, 1), 5 = (2, 1); for the fp8 append the same bits read: bit 12 = waves that convert a whole
  *   row, bit 13 = waves that convert 512 elements (0 = by launch size);
  * bits 16-19: log2 of the blocks per plane visit of pack / unpack (15 = plain order);
@@ -30,8 +30,8 @@ extern "C" {
  *   per XCD (default: chosen per launch by kind, table length, tiles per chunk and plane size);
  * bit 28: the paged-layout append always through the general kernel (256-thread workgroups, block barrier) instead of
  *   the kernel of one-wave workgroups that the usual shapes take;
- * bits 29-30: column width of the one-wave paged-layout append (1 = 128 row elements, 2 = 32, 3 = 256; 0 = by launch
- *   size); with it bits 20-21: 1 = K and V of a column in one wave, 2 = in two waves (0 = by launch size).
+ * bits 29-30: column width of the one-wave paged-layout append (1 = 128 row elements, 2 = 32, 3 = 256, or 64 with bit 22
+ *   set; 0 = by launch size); with it bits 20-21: 1 = K and V of a column in one wave, 2 = in two waves (0 = by launch size).
  * Process-wide, not thread-safe. Returns the previous value. */
 int emm_hook_set_move_variant(int variant);
 
