@@ -1348,6 +1348,37 @@ def test_paged_append_all_layers_on_both_sides_of_its_rules(cache, H, D, bs, T, 
         assert same_bits(kcs[l], kc) and same_bits(vcs[l], vc), f"layer {l}"
 
 
+# 16-bit launches of 448 pieces and more: V of a single token is stored by one policy beside a token of its 16-slot window, by
+# another alone. (H, D, bs, rows of the prompts' ends, step between slots): -1 walks a block backwards, 16 puts every token alone
+@pytest.mark.parametrize("layers", [1, 3])
+@pytest.mark.parametrize("H,D,bs,q,step", [(4, 128, 16, 15, 1), (4, 128, 32, 1, 1), (5, 104, 16, 2, 1), (9, 120, 64, 11, 1),
+                                           (4, 128, 32, 20, 1), (4, 128, 16, 15, -1), (4, 128, 64, 4, 16)])
+def test_paged_append_of_many_short_prompts(layers, H, D, bs, q, step):
+    T = 1800
+    NB = T // q + 40
+    say(f"paged append, short prompts: layers={layers} H={H} D={D} bs={bs} q={q} step={step}")
+    g = torch.Generator().manual_seed(T + q)
+    slots = []
+    for n, b in enumerate(torch.randperm(NB, generator=g).tolist()):
+        first = int(torch.randint(bs - (q - 1) * abs(step), (1,), generator=g))
+        run = [b * bs + first + i * abs(step) for i in range(q)]
+        slots += run if step > 0 else run[::-1]
+        if n % 7 == 3: slots.append(-1)  # a padded entry behind a prompt
+    slots = torch.tensor(slots[:T], dtype=torch.long)
+    assert len(slots) == T and (T + 15) // 16 * ((H * D + 127) // 128) >= 448
+    keys, values = ([torch.randn((T, H, D), generator=g).to(torch.bfloat16) for _ in range(layers)] for _ in range(2))
+    caches = [paged_caches_cpu(NB, H, D, bs, torch.bfloat16, fill_mod=31 + l) for l in range(layers)]
+    kcs, vcs = ([c[i].to(DEV) for c in caches] for i in range(2))
+    if layers == 1:
+        cache_ops.reshape_and_cache(keys[0].to(DEV), values[0].to(DEV), kcs[0], vcs[0], slots.to(DEV))
+    else:
+        one = torch.ones(layers)
+        cache_ops.paged_layered_append([k.to(DEV) for k in keys], [v.to(DEV) for v in values], kcs, vcs, "auto", one, one)(slots.to(DEV))
+    for l, (kc, vc) in enumerate(caches):
+        orc.c_reshape_and_cache_paged(keys[l], values[l], kc, vc, slots)
+        assert same_bits(kcs[l], kc) and same_bits(vcs[l], vc), f"layer {l}"
+
+
 @pytest.mark.parametrize("T", [6656, 6657])
 def test_paged_append_fp8_of_many_layers_on_both_sides_of_its_rule(T):
     """96 layers of 256 elements: 832 pieces a layer take the one-wave kernel, 834 (80000 in all) the general one."""
