@@ -1305,9 +1305,9 @@ def test_paged_append_every_dispatched_wave_shape(cache, H, D, bs, T, phase):
 
 
 # per layer, 16-bit caches: single tokens written through up to 128 pieces
-# fp8: the general kernel up to 1024 pieces and from 1440 to 2048
+# fp8: the general kernel up to 1024 pieces and from 1440 to 2048, but for tile counts of up to 256 that are powers of two
 @pytest.mark.parametrize("cache,H,D,bs,T,phase", [("fp8", 20, 128, 16, 1136, 3), ("fp8_sat", 20, 128, 16, 1137, 0), ("fp8_sat", 20, 128, 16, 1632, 7),
-                                                  ("fp8", 20, 128, 32, 1633, 2), ("auto", 5, 104, 16, 400, 3), ("auto", 5, 104, 16, 401, 0),
+                                                  ("fp8", 20, 128, 32, 1633, 2), ("fp8", 13, 128, 16, 2048, 1), ("fp8_sat", 13, 128, 16, 2049, 0), ("auto", 5, 104, 16, 400, 3), ("auto", 5, 104, 16, 401, 0),
                                                   ("auto", 9, 120, 32, 224, 1), ("auto", 9, 120, 32, 225, 14)])
 def test_paged_append_on_both_sides_of_its_rules(cache, H, D, bs, T, phase):
     test_paged_append_every_dispatched_wave_shape(cache, H, D, bs, T, phase)
