@@ -20,8 +20,11 @@ from ._lib import (EMM_DTYPE_BF16, EMM_DTYPE_F16, EMM_FP8_SATURATE, EMM_MAX_INLI
 IndexLike = Union[Sequence[int], np.ndarray, torch.Tensor]
 
 
-# the current GPU's index, and the hipStream_t of torch's current stream on a GPU given by its index
+# the current GPU's index, the number of GPUs, and the hipStream_t of torch's current stream on a GPU given by its index. The
+# number is the HIP runtime's: torch.cuda.device_count() starts the system-management library for it, which opens the devices
+# a second time beside the runtime.
 _get_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+_device_count = getattr(torch._C, "_cuda_getDeviceCount", torch.cuda.device_count)
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", lambda index: torch.cuda.current_stream(index).cuda_stream)
 
 
@@ -136,7 +139,7 @@ class PoolView:
         self.device = first.device if pinned_host_for is None else torch.device(pinned_host_for)
         # the GPU's index where a launch has to ask which one is current (``_elsewhere`` without its cost for a single GPU:
         # pack and unpack run in front of kernels of a few microseconds)
-        self.one_of_several = self.device.index if torch.cuda.device_count() > 1 else None
+        self.one_of_several = self.device.index if _device_count() > 1 else None
         self.on_host = pinned_host_for is not None
         self.dtype = first.dtype
         self.elem_bytes = first.element_size()

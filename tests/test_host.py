@@ -681,7 +681,11 @@ class OtherGpuIsCurrent:
                 return entry
 
         monkeypatch.setattr(torch.cuda, "device", Device)
-        monkeypatch.setattr(torch.cuda, "device_count", lambda: 2)
+        def starts_the_management_library():
+            raise AssertionError("an operator asked torch.cuda for the number of GPUs")
+
+        monkeypatch.setattr(torch.cuda, "device_count", starts_the_management_library)
+        monkeypatch.setattr(kv_ops, "_device_count", lambda: 2, raising=False)
         monkeypatch.setattr(kv_ops, "_get_device", lambda: rig.current)
         monkeypatch.setattr(kv_ops, "_raw_stream", lambda index: 0)
         monkeypatch.setattr(_lib, "_lib", Lib())
