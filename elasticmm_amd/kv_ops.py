@@ -138,7 +138,7 @@ class PoolView:
         self.layers: List[torch.Tensor] = layers
         self.device = first.device if pinned_host_for is None else torch.device(pinned_host_for)
         # the GPU's index where a launch has to ask which one is current (``_elsewhere`` without its cost for a single GPU:
-        # pack and unpack run in front of kernels of a few microseconds)
+        # the block moves run in front of kernels of a few microseconds)
         self.one_of_several = self.device.index if _device_count() > 1 else None
         self.on_host = pinned_host_for is not None
         self.dtype = first.dtype
@@ -276,7 +276,7 @@ def kv_migrate(src: PoolView, src_indices: IndexLike, dst: PoolView, dst_indices
     """``dst[l][:, dst_idx[j]] = src[l][:, src_idx[j]]`` in one launch, no staging buffer (``strict``: as in
     ``kv_pack``, for either table)."""
     lib = _lib.load()
-    if _elsewhere(src.device):
+    if src.one_of_several is not None and src.one_of_several != _get_device():
         with torch.cuda.device(src.device):
             return kv_migrate(src, src_indices, dst, dst_indices, strict)
     if strict:
@@ -315,7 +315,7 @@ def copy_blocks(pool: PoolView, block_mapping: Union[torch.Tensor, Sequence[Sequ
     """All layers: ``pool[:, dst] = pool[:, src]`` for the (src, dst) rows of ``block_mapping`` (``strict``: a
     device mapping is validated first, as in ``kv_pack``; without it pairs with an id out of range are skipped)."""
     lib = _lib.load()
-    if _elsewhere(pool.device):
+    if pool.one_of_several is not None and pool.one_of_several != _get_device():
         with torch.cuda.device(pool.device):
             return copy_blocks(pool, block_mapping, strict)
     if strict and isinstance(block_mapping, torch.Tensor) and block_mapping.is_cuda:
@@ -359,7 +359,7 @@ def kv_unpack_dequant_fp8(pool: PoolView, block_indices: IndexLike, packed_fp8: 
     """Scatter an fp8-e4m3fn transfer buffer ``[L, 2, n, ...]`` into a bf16/f16 pool,
     ``out = rne16(float(q) * scale)`` with per-layer K and V scales."""
     lib = _lib.load()
-    if _elsewhere(pool.device):
+    if pool.one_of_several is not None and pool.one_of_several != _get_device():
         with torch.cuda.device(pool.device):
             return kv_unpack_dequant_fp8(pool, block_indices, packed_fp8, k_scales, v_scales)
     _require_gpu(packed_fp8, "kv_unpack_dequant_fp8")
