@@ -819,7 +819,7 @@ def paged_append_bench(kv, NB, bs, H, D, dev, T=8448, decode=256, k_scales=None,
     ce = kv[0].element_size()
     fp8 = k_scales is not None
     cache_dtype = "fp8" if fp8 else "auto"
-    kernel = "emm_append_paged_kernel" if fp8 else "emm_append_paged_wave_kernel"
+    kernel = "emm_append_paged_wave_kernel"
     x = 16 // ce
     g = torch.Generator(device=dev).manual_seed(4)
     blocks = torch.randperm(NB, device=dev, generator=g)

@@ -1268,8 +1268,7 @@ def test_paged_append_fp8(dtype, phase, T):
     assert int((vc_g.cpu() & 0x7F).eq(0x7F).sum()) > (100 if T >= 2000 else 3)
 
 
-# (cache, H, D, bs, T, phase): the one-wave kernel's shapes change at 192 and 448 pieces (16-bit: 32, 64, 128 row elements
-# per wave), at 256 and past 1024 (fp8: 32, general kernel, 64); pieces = ceil(T / 16) * ceil(H * D / 128)
+# (cache, H, D, bs, T, phase): steps of 1 to 3000 pieces; pieces = ceil(T / 16) * ceil(H * D / 128)
 @pytest.mark.parametrize("cache,H,D,bs,T,phase", [
     ("auto", 4, 128, 16, 752, 0), ("auto", 4, 128, 16, 753, 3), ("auto", 5, 104, 16, 700, 7), ("auto", 3, 72, 32, 1100, 1),
     ("auto", 4, 128, 16, 1776, 5), ("auto", 4, 128, 16, 1777, 11), ("auto", 5, 104, 64, 1500, 2),
@@ -1304,8 +1303,7 @@ def test_paged_append_every_dispatched_wave_shape(cache, H, D, bs, T, phase):
     assert same_bits(kc_g, kc) and same_bits(vc_g, vc)
 
 
-# per layer, 16-bit caches: single tokens written through up to 128 pieces
-# fp8: the general kernel up to 1024 pieces and from 1440 to 2048, but for tile counts of up to 256 that are powers of two
+# per layer: tile counts of up to 256 that are powers of two, and their neighbours; few and many pieces
 @pytest.mark.parametrize("cache,H,D,bs,T,phase", [("fp8", 20, 128, 16, 1136, 3), ("fp8_sat", 20, 128, 16, 1137, 0), ("fp8_sat", 20, 128, 16, 1632, 7),
                                                   ("fp8", 20, 128, 32, 1633, 2), ("fp8", 13, 128, 16, 2048, 1), ("fp8_sat", 13, 128, 16, 2049, 0), ("auto", 5, 104, 16, 400, 3), ("auto", 5, 104, 16, 401, 0),
                                                   ("auto", 9, 120, 32, 224, 1), ("auto", 9, 120, 32, 225, 14)])
@@ -1313,8 +1311,7 @@ def test_paged_append_on_both_sides_of_its_rules(cache, H, D, bs, T, phase):
     test_paged_append_every_dispatched_wave_shape(cache, H, D, bs, T, phase)
 
 
-# all layers in one launch: pieces = ceil(T / 16) * ceil(H * D / 128). 16-bit: single tokens written through below 448 pieces,
-# non-temporal from there; fp8: the general kernel below 256 pieces, 64-element waves from there
+# all layers in one launch: pieces = ceil(T / 16) * ceil(H * D / 128), few and many; rows that 64-element waves cut evenly and not
 @pytest.mark.parametrize("cache,H,D,bs,T,phase", [
     ("auto", 5, 104, 16, 1424, 3), ("auto", 5, 104, 16, 1425, 0), ("auto", 5, 104, 32, 3680, 1), ("auto", 9, 120, 16, 784, 2),
     ("auto", 9, 120, 64, 785, 5), ("auto", 2, 40, 16, 33, 6),
@@ -1348,8 +1345,7 @@ def test_paged_append_all_layers_on_both_sides_of_its_rules(cache, H, D, bs, T, 
         assert same_bits(kcs[l], kc) and same_bits(vcs[l], vc), f"layer {l}"
 
 
-# 16-bit launches of 448 pieces and more: V of a single token is stored by one policy beside a token of its 16-slot window, by
-# another alone. (H, D, bs, rows of the prompts' ends, step between slots): -1 walks a block backwards, 16 puts every token alone
+# V of a single token is stored by one policy beside a token of its 16-slot window, by another alone. (H, D, bs, rows of the prompts' ends, step between slots): -1 walks a block backwards, 16 puts every token alone
 @pytest.mark.parametrize("layers", [1, 3])
 @pytest.mark.parametrize("H,D,bs,q,step", [(4, 128, 16, 15, 1), (4, 128, 32, 1, 1), (5, 104, 16, 2, 1), (9, 120, 64, 11, 1),
                                            (4, 128, 32, 20, 1), (4, 128, 16, 15, -1), (4, 128, 64, 4, 16)])
@@ -1377,6 +1373,58 @@ def test_paged_append_of_many_short_prompts(layers, H, D, bs, q, step):
     for l, (kc, vc) in enumerate(caches):
         orc.c_reshape_and_cache_paged(keys[l], values[l], kc, vc, slots)
         assert same_bits(kcs[l], kc) and same_bits(vcs[l], vc), f"layer {l}"
+
+
+# the wave shapes change past 32 pieces, at 320 and 768 (16-bit), at 2600 with rows of up to 512, up to 1024 and more elements,
+# at 512 and 1600 (fp8)
+@pytest.mark.parametrize("cache,H,D,bs,T,phase", [
+    ("auto", 4, 128, 16, 128, 3), ("auto", 4, 128, 16, 129, 5), ("auto", 5, 104, 16, 1008, 2), ("auto", 5, 104, 16, 1009, 0), ("auto", 4, 128, 32, 3056, 9),
+    ("auto", 4, 128, 16, 3057, 1), ("auto", 9, 120, 16, 1360, 0), ("auto", 9, 120, 16, 1361, 4), ("auto", 13, 128, 16, 3184, 7), ("auto", 13, 128, 16, 3185, 7),
+    ("auto", 4, 128, 16, 10384, 1), ("auto", 4, 128, 16, 10385, 0), ("auto", 1, 64, 16, 12400, 6), ("fp8", 4, 128, 16, 128, 0), ("fp8_sat", 4, 128, 16, 129, 2),
+    ("fp8", 4, 128, 16, 2032, 3), ("fp8_sat", 4, 128, 16, 2033, 3), ("fp8", 10, 128, 16, 2544, 11), ("fp8_sat", 10, 128, 32, 2545, 0)])
+def test_paged_append_on_both_sides_of_its_wave_shapes(cache, H, D, bs, T, phase):
+    test_paged_append_every_dispatched_wave_shape(cache, H, D, bs, T, phase)
+
+
+# (cache, H, D, bs, short, prompt): one case per launch shape, whole column widths and not; `short`: the first tokens only
+@pytest.mark.parametrize("cache,H,D,bs,short,prompt", [
+    ("auto", 2, 64, 16, 500, 0), ("auto", 4, 128, 16, 0, 0), ("auto", 5, 104, 32, 0, 0), ("auto", 8, 128, 16, 0, 16), ("auto", 9, 72, 64, 0, 1000),
+    ("auto", 4, 128, 16, 0, 3000), ("auto", 4, 120, 16, 0, 3005), ("auto", 8, 128, 16, 0, 1607), ("auto", 9, 120, 16, 0, 1600),
+    ("auto", 12, 128, 16, 0, 2800), ("auto", 11, 120, 32, 0, 3300), ("auto", 1, 64, 16, 0, 12500),
+    ("fp8", 2, 64, 16, 500, 0), ("fp8_sat", 4, 128, 16, 0, 0), ("fp8", 5, 112, 32, 0, 33), ("fp8_sat", 8, 128, 16, 0, 900), ("fp8", 9, 112, 16, 0, 1000),
+    ("fp8", 8, 128, 16, 0, 3001), ("fp8_sat", 9, 112, 64, 0, 3000)])
+def test_paged_append_partial_runs_at_every_place(cache, H, D, bs, short, prompt):
+    """Runs of every length at every offset of a 16-slot window, in any place of the token tiles, between single tokens and
+    behind a prompt of whole windows."""
+    say(f"paged append, partial runs: {cache} H={H} D={D} bs={bs} short={short} prompt={prompt}")
+    g = torch.Generator().manual_seed(H * D + prompt)
+    places = [(off, n) for n in range(1, 17) for off in range(17 - n)]
+    NB = len(places) + (prompt + bs - 1) // bs + 1
+    blocks = torch.randperm(NB, generator=g).tolist()
+    slots = [blocks[i // bs] * bs + i % bs for i in range(prompt)]
+    blocks = blocks[(prompt + bs - 1) // bs:]
+    for i in torch.randperm(len(places), generator=g).tolist():
+        off, n = places[i]
+        first = blocks.pop() * bs + 16 * int(torch.randint(bs // 16, (1,), generator=g)) + off
+        slots += range(first, first + n)
+    slots = torch.tensor(slots[:short] if short else slots, dtype=torch.long)
+    T = len(slots)
+    dtype = torch.bfloat16
+    key, value = ((torch.randn((T, H, D), generator=g) * 30).to(dtype) for _ in range(2))
+    kc, vc = paged_caches_cpu(NB, H, D, bs, dtype if cache == "auto" else torch.uint8)
+    kc_g, vc_g = kc.to(DEV), vc.to(DEV)
+    if cache == "auto":
+        cache_ops.reshape_and_cache(key.to(DEV), value.to(DEV), kc_g, vc_g, slots.to(DEV))
+        orc.c_reshape_and_cache_paged(key, value, kc, vc, slots)
+    else:
+        ks, vs = torch.tensor([0.05]), torch.tensor([0.31])
+        cache_ops.reshape_and_cache(key.to(DEV), value.to(DEV), kc_g, vc_g, slots.to(DEV), cache, ks.to(DEV), vs.to(DEV))
+        if cache == "fp8_sat":  # the bytes of the saturating cast, placed by the byte-copying reference
+            k8, v8 = (torch.from_numpy(orc.c_quant_fp8_sat(x, float(sc)).reshape(T, H, D).copy()) for x, sc in ((key, ks), (value, vs)))
+            orc.ref_reshape_and_cache_paged(k8, v8, kc, vc, slots)
+        else:
+            orc.c_reshape_and_cache_paged(key, value, kc, vc, slots, float(ks), float(vs))
+    assert same_bits(kc_g, kc) and same_bits(vc_g, vc)
 
 
 @pytest.mark.parametrize("bs,seqs,chunk,pad", [(16, 1, 0, 0), (16, 24, 0, 3), (16, 239, 0, 0), (16, 240, 0, 0), (12, 400, 1000, 7),
