@@ -841,7 +841,7 @@ def paged_append_bench(kv, NB, bs, H, D, dev, T=8448, decode=256, k_scales=None,
             cache_ops.reshape_and_cache(keys[l], values[l], kcs[l], vcs[l], slots, cache_dtype, ks[l], vs[l])
 
     def entry(ms, launches):
-        return rec(step_bytes, ms, launches, kernel, tokens_per_s=round(T / (ms * 1e-3)))
+        return rec(step_bytes, ms, launches, kernel if launches == 1 else per_layer_kernel, tokens_per_s=round(T / (ms * 1e-3)))
 
     res = {"T": T, "decode_tokens": decode, "layers": L}
     med, _ = timed(per_layer, 20)
@@ -941,14 +941,15 @@ def append_bench(kv, NB, bs, H, D, k_scales, v_scales, dev, T=8448):
     step_bytes = L * (valid * 2 * row * (2 + kv[0].element_size()) + 8 * T)
     ks = [None] * L if not fp8 else [k_scales[l:l + 1] for l in range(L)]
     vs = [None] * L if not fp8 else [v_scales[l:l + 1] for l in range(L)]
-    kernel = "emm_append_fp8_kernel" if fp8 else "emm_append_kernel"
+    kernel = "emm_append_fp8_kernel" if fp8 else "emm_append_kernel"  # one launch for all layers
+    per_layer_kernel = kernel if fp8 else "emm_append_tile_kernel"
 
     def per_layer():
         for l in range(L):
             cache_ops.reshape_and_cache_flash(keys[l], values[l], kv[l][0], kv[l][1], slots, mode, ks[l], vs[l])
 
     def entry(ms, launches):
-        return rec(step_bytes, ms, launches, kernel, tokens_per_s=round(valid / (ms * 1e-3)))
+        return rec(step_bytes, ms, launches, kernel if launches == 1 else per_layer_kernel, tokens_per_s=round(valid / (ms * 1e-3)))
 
     def graphed(fn):
         graph = torch.cuda.CUDAGraph()
@@ -977,7 +978,7 @@ def append_bench(kv, NB, bs, H, D, k_scales, v_scales, dev, T=8448):
     # without the appends; the difference per layer is what the forward pays for an append.
     if APPEND_CONTEXT:
         res["in_context"] = append_in_context(keys, values, kv, slots, mode, ks, vs, entry, graphed, step_bytes, valid,
-                                              kernel, T, H, D, L, dev, g)
+                                              per_layer_kernel, T, H, D, L, dev, g)
     # a decode step: 256 tokens, one per sequence, per-layer launches from a HIP graph (the most frequent step of a
     # serving loop; 1 MB per launch, so the figure of merit is microseconds per launch against the empty launch)
     Td = 256

@@ -702,8 +702,8 @@ def test_cfg3_append_reduced_pool():
 
 @pytest.mark.parametrize("T", [1, 3, 1536, 1537, 2051, 6144, 6145, 6147])
 def test_append_token_counts_around_the_wave_shape_thresholds(T):
-    """The per-layer append picks 1, 2 or 4 token rows per wave from the token count: both sides of each
-    threshold, and counts that leave the last wave partly empty."""
+    """The per-layer append picks the rows of a wave from the token count and the bytes: both sides of thresholds, and
+    counts that leave the last wave partly empty."""
     NB, bs, H, D = 512, 16, 4, 128
     slots = make_slots(NB * bs, T, T, pad_frac=0.05)
     g = torch.Generator().manual_seed(T)
@@ -1455,8 +1455,8 @@ def test_slot_mapping_on_the_device(bs, seqs, chunk, pad):
 @pytest.mark.parametrize("cache,H,D", [("auto", 4, 128), ("auto", 8, 128), ("auto", 1, 8), ("auto", 5, 104), ("fp8", 4, 128),
                                        ("fp8", 5, 104), ("fp8_sat", 1, 8), ("fp8_sat", 9, 120), ("fp8", 7, 72)])
 def test_flash_append_on_both_sides_of_its_launch_rules(cache, H, D, T):
-    """Per layer: rows per wave and store policy change past 1536 and 3072 tokens and with rows longer than 1 KiB; fp8 rows
-    of at most 512 elements take the thin waves."""
+    """Per layer: rows per wave, pieces of a row and store policy change with the tokens, the row and the bytes; fp8 rows of at
+    most 512 elements take the thin waves."""
     NB, bs = 250, 16
     g = torch.Generator().manual_seed(T + H)
     wide = (torch.randn((T, 2 * H * D), generator=g) * 20).to(torch.bfloat16)
@@ -1487,6 +1487,49 @@ def test_flash_append_on_both_sides_of_its_launch_rules(cache, H, D, T):
 @pytest.mark.parametrize("cache,H,D,T", [("fp8", 9, 120, 2777), ("fp8_sat", 17, 128, 1600), ("fp8", 16, 128, 1600)])
 def test_flash_append_fp8_store_policies(cache, H, D, T):
     test_flash_append_on_both_sides_of_its_launch_rules(cache, H, D, T)
+
+
+# one call per layer, every shape of the tile kernels: tokens that fill a wave's rows and do not, rows that fill its pieces, leave some
+# empty or do not end on a 128-byte line, both sides of the rules on tokens and bytes
+@pytest.mark.parametrize("cache,H,D,T", [
+    ("auto", 1, 64, 768), ("auto", 1, 64, 769), ("auto", 8, 72, 1), ("auto", 8, 128, 15), ("auto", 16, 128, 33), ("auto", 1, 48, 1000),
+    ("auto", 4, 128, 2559), ("auto", 4, 128, 2560), ("auto", 4, 128, 3583), ("auto", 4, 128, 3584), ("auto", 4, 128, 5119),
+    ("auto", 4, 128, 5120), ("auto", 8, 128, 2047), ("auto", 8, 128, 2051), ("auto", 2, 128, 9215), ("auto", 2, 128, 9217),
+    ("auto", 3, 64, 12289), ("auto", 9, 128, 1820), ("auto", 9, 128, 1825), ("auto", 5, 64, 7375), ("auto", 1, 72, 1003),
+    ("auto", 1, 120, 8737), ("auto", 1, 120, 8739), ("auto", 2, 100, 1001), ("auto", 2, 100, 11801), ("auto", 5, 104, 1),
+    ("auto", 5, 104, 6), ("auto", 5, 104, 4035), ("auto", 3, 104, 7567),
+    ("fp8", 1, 128, 3072), ("fp8", 1, 128, 3073), ("fp8_sat", 1, 40, 3075), ("fp8", 3, 64, 3079), ("fp8_sat", 2, 128, 8191),
+    ("fp8", 2, 128, 8193), ("fp8_sat", 4, 128, 4095), ("fp8", 4, 128, 4101), ("fp8", 4, 128, 8192), ("fp8", 5, 40, 3081),
+    ("fp8", 9, 120, 1), ("fp8_sat", 9, 120, 1023), ("fp8", 9, 120, 1025), ("fp8", 17, 128, 963), ("fp8_sat", 17, 128, 965)])
+def test_flash_append_every_tile_shape(cache, H, D, T):
+    NB, bs = T // 12 + 9, 16
+    dtype = torch.float16 if T % 2 else torch.bfloat16
+    say(f"flash append, tile shapes: {cache} H={H} D={D} T={T} {dtype}")
+    g = torch.Generator().manual_seed(T + H)
+    pad = 8 * (T % 3)  # extra elements per source row; whole rows apart, and views of a wider projection
+    wide = (torch.randn((T, 2 * H * D + pad), generator=g) * 20).to(dtype)
+    key, value = (wide[:, i * H * D:(i + 1) * H * D].reshape(T, H, D).contiguous() for i in range(2))
+    slots = torch.randperm(NB * bs, generator=g)[:T]
+    if T > 6:
+        slots[3::17] = -1
+        slots[5::29] = NB * bs + torch.arange(len(slots[5::29])) * 2 ** 31  # past the cache, past 32 bits: skipped
+    kc = torch.full((NB, bs, H, D), 5, dtype=dtype if cache == "auto" else torch.uint8)
+    vc = kc.clone()
+    kc_g, vc_g, wide_g = kc.to(DEV), vc.to(DEV), wide.to(DEV)
+    key_g, value_g = (wide_g[:, i * H * D:(i + 1) * H * D].view(T, H, D) for i in range(2))
+    inside = torch.where(slots < NB * bs, slots, -1)
+    if cache == "auto":
+        cache_ops.reshape_and_cache_flash(key_g, value_g, kc_g, vc_g, slots.to(DEV))
+        orc.c_reshape_and_cache(key, value, kc, vc, inside)
+    else:
+        ks, vs = torch.tensor([0.05]), torch.tensor([0.11])
+        cache_ops.reshape_and_cache_flash(key_g, value_g, kc_g, vc_g, slots.to(DEV), cache, ks.to(DEV), vs.to(DEV))
+        if cache == "fp8_sat":
+            k8, v8 = (torch.from_numpy(orc.c_quant_fp8_sat(x, float(sc)).reshape(T, H, D).copy()) for x, sc in ((key, ks), (value, vs)))
+            orc.c_reshape_and_cache(k8, v8, kc, vc, inside)
+        else:
+            orc.c_reshape_and_cache_fp8(key, value, kc, vc, inside, float(ks), float(vs))
+    assert same_bits(kc_g, kc) and same_bits(vc_g, vc)
 
 
 @pytest.mark.parametrize("layout", ["flash", "paged"])
