@@ -72,7 +72,7 @@ int unpack_dequant(void *const *layer_ptrs, int num_layers, int64_t num_blocks,
     const dim3 grid = grouped ? dim3((uint32_t)tpc, (uint32_t)((2 * num_layers) << 8), (uint32_t)((ny + 255) >> 8))
                               : dim3((uint32_t)tpc, (uint32_t)ny, (uint32_t)(2 * num_layers));
 #define EMM_DQ_LAUNCH(DT, G, IN, IDS) \
-  emm_unpack_dequant_fp8_kernel<DT, G, IN><<<grid, kThreads, 0, s>>>(packed, idx, k_scales, v_scales, stride, \
+  enqueue(emm_unpack_dequant_fp8_kernel<DT, G, IN>, grid, kThreads, s, packed, idx, k_scales, v_scales, stride, \
       (uint32_t)chunk_elems, (uint32_t)num_blocks, (uint32_t)ny, 8u | remap, t, IDS)
     if (host_idx) { // at most EMM_MAX_INLINE_IDS blocks: never grouped
       InlineIds ids;
@@ -195,10 +195,10 @@ int emm_stream_copy(const void *src, void *dst, int64_t nbytes, emm_stream_t str
   const char *a = (const char *)src;
   char *b = (char *)dst;
   switch (vec) {
-  case 16: emm_stream_copy_kernel<u32x4, 1, 1><<<grid, kThreads, 0, s>>>(a, b, nbytes); break;
-  case 4: emm_stream_copy_kernel<uint32_t, 4, 0><<<grid, kThreads, 0, s>>>(a, b, nbytes); break;
-  case 2: emm_stream_copy_kernel<uint16_t, 4, 0><<<grid, kThreads, 0, s>>>(a, b, nbytes); break;
-  default: emm_stream_copy_kernel<uint8_t, 4, 0><<<grid, kThreads, 0, s>>>(a, b, nbytes); break;
+  case 16: enqueue(emm_stream_copy_kernel<u32x4, 1, 1>, grid, kThreads, s, a, b, nbytes); break;
+  case 4: enqueue(emm_stream_copy_kernel<uint32_t, 4, 0>, grid, kThreads, s, a, b, nbytes); break;
+  case 2: enqueue(emm_stream_copy_kernel<uint16_t, 4, 0>, grid, kThreads, s, a, b, nbytes); break;
+  default: enqueue(emm_stream_copy_kernel<uint8_t, 4, 0>, grid, kThreads, s, a, b, nbytes); break;
   }
   return check_launch("emm_stream_copy");
 }
@@ -363,7 +363,7 @@ int emm_slot_mapping(const int64_t *host_starts, const int64_t *host_offsets, co
   const bool pad = pad_to > total;
   if (seqs == 0 && !pad) return EMM_OK;
   const int64_t strips = (longest + 255) / 256;
-  emm_slot_mapping_kernel<<<dim3((uint32_t)(seqs + (pad ? 1 : 0)), (uint32_t)(strips < 64 ? strips : 64)), 256, 0, as_stream(stream)>>>(
+  enqueue(emm_slot_mapping_kernel, dim3((uint32_t)(seqs + (pad ? 1 : 0)), (uint32_t)(strips < 64 ? strips : 64)), 256, as_stream(stream),
       out, (uint32_t)seqs, (uint32_t)block_size, (uint32_t)pad_to, t);
   return check_launch(what);
 }
@@ -410,10 +410,10 @@ int emm_concat_rows(const void *const *srcs, const int64_t *nbytes, int n, void 
   dim3 grid((uint32_t)tiles);
   hipStream_t s = as_stream(stream);
   switch (al) {
-  case 16: emm_concat_rows_kernel<u32x4, 1><<<grid, kThreads, 0, s>>>(p); break;
-  case 4: emm_concat_rows_kernel<uint32_t, 4><<<grid, kThreads, 0, s>>>(p); break;
-  case 2: emm_concat_rows_kernel<uint16_t, 4><<<grid, kThreads, 0, s>>>(p); break;
-  default: emm_concat_rows_kernel<uint8_t, 4><<<grid, kThreads, 0, s>>>(p); break;
+  case 16: enqueue(emm_concat_rows_kernel<u32x4, 1>, grid, kThreads, s, p); break;
+  case 4: enqueue(emm_concat_rows_kernel<uint32_t, 4>, grid, kThreads, s, p); break;
+  case 2: enqueue(emm_concat_rows_kernel<uint16_t, 4>, grid, kThreads, s, p); break;
+  default: enqueue(emm_concat_rows_kernel<uint8_t, 4>, grid, kThreads, s, p); break;
   }
   return check_launch(what);
 }
