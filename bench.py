@@ -841,7 +841,7 @@ def paged_append_bench(kv, NB, bs, H, D, dev, T=8448, decode=256, k_scales=None,
             cache_ops.reshape_and_cache(keys[l], values[l], kcs[l], vcs[l], slots, cache_dtype, ks[l], vs[l])
 
     def entry(ms, launches):
-        return rec(step_bytes, ms, launches, kernel if launches == 1 else per_layer_kernel, tokens_per_s=round(T / (ms * 1e-3)))
+        return rec(step_bytes, ms, launches, kernel, tokens_per_s=round(T / (ms * 1e-3)))
 
     res = {"T": T, "decode_tokens": decode, "layers": L}
     med, _ = timed(per_layer, 20)
