@@ -1494,7 +1494,8 @@ def test_flash_append_fp8_store_policies(cache, H, D, T):
 @pytest.mark.parametrize("cache,H,D,T", [
     ("auto", 1, 64, 768), ("auto", 1, 64, 769), ("auto", 8, 72, 1), ("auto", 8, 128, 15), ("auto", 16, 128, 33), ("auto", 1, 48, 1000),
     ("auto", 4, 128, 2559), ("auto", 4, 128, 2560), ("auto", 4, 128, 3583), ("auto", 4, 128, 3584), ("auto", 4, 128, 5119),
-    ("auto", 4, 128, 5120), ("auto", 8, 128, 2047), ("auto", 8, 128, 2051), ("auto", 2, 128, 9215), ("auto", 2, 128, 9217),
+    ("auto", 4, 128, 5120), ("auto", 4, 128, 7167), ("auto", 4, 128, 7171), ("auto", 4, 128, 9215), ("auto", 4, 128, 9216),
+    ("auto", 8, 128, 2047), ("auto", 8, 128, 2051), ("auto", 2, 128, 9215), ("auto", 2, 128, 9217),
     ("auto", 3, 64, 12289), ("auto", 9, 128, 1820), ("auto", 9, 128, 1825), ("auto", 5, 64, 7375), ("auto", 1, 72, 1003),
     ("auto", 1, 120, 8737), ("auto", 1, 120, 8739), ("auto", 2, 100, 1001), ("auto", 2, 100, 11801), ("auto", 5, 104, 1),
     ("auto", 5, 104, 6), ("auto", 5, 104, 4035), ("auto", 3, 104, 7567),
