@@ -1533,6 +1533,12 @@ def test_flash_append_every_tile_shape(cache, H, D, T):
     assert same_bits(kc_g, kc) and same_bits(vc_g, vc)
 
 
+# both ends of the launches that take four whole rows a wave
+@pytest.mark.parametrize("H,D,T", [(5, 64, 3583), (5, 64, 3585), (7, 64, 4607), (7, 64, 4609), (4, 128, 4607), (4, 128, 4608)])
+def test_flash_append_around_four_rows_a_wave(H, D, T):
+    test_flash_append_every_tile_shape("auto", H, D, T)
+
+
 # one call of more rows than a tile shape's grid holds (8 rows x 65535, 4 x 65535) and of the last that it does hold
 @pytest.mark.parametrize("H,D,T", [(1, 8, 262141), (1, 8, 524280), (1, 8, 524281), (1, 16, 262145), (1, 72, 262145)])
 def test_flash_append_of_more_tokens_than_a_grid_holds(H, D, T):
