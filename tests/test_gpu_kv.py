@@ -1539,6 +1539,12 @@ def test_flash_append_around_four_rows_a_wave(H, D, T):
     test_flash_append_every_tile_shape("auto", H, D, T)
 
 
+# fp8 rows that fill a tile wave once or twice: both ends of the tile kernel's range
+@pytest.mark.parametrize("cache,T", [("fp8", 4097), ("fp8_sat", 6143), ("fp8", 6144), ("fp8_sat", 6149)])
+def test_flash_append_fp8_rows_of_512_on_both_sides_of_their_rule(cache, T):
+    test_flash_append_every_tile_shape(cache, 4, 128, T)
+
+
 # one call of more rows than a tile shape's grid holds (8 rows x 65535, 4 x 65535) and of the last that it does hold
 @pytest.mark.parametrize("H,D,T", [(1, 8, 262141), (1, 8, 524280), (1, 8, 524281), (1, 16, 262145), (1, 72, 262145)])
 def test_flash_append_of_more_tokens_than_a_grid_holds(H, D, T):
