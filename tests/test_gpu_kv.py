@@ -1386,6 +1386,12 @@ def test_paged_append_on_both_sides_of_its_wave_shapes(cache, H, D, bs, T, phase
     test_paged_append_every_dispatched_wave_shape(cache, H, D, bs, T, phase)
 
 
+# rows of more than 1024 elements from 4000 pieces: 128-wide waves that do not hold their stores back, whole columns and not
+@pytest.mark.parametrize("H,D,bs,T,phase", [(16, 128, 16, 3984, 3), (16, 128, 16, 3985, 0), (17, 120, 32, 4007, 5), (32, 128, 16, 2000, 11)])
+def test_paged_append_of_long_rows_around_its_widest_launches(H, D, bs, T, phase):
+    test_paged_append_every_dispatched_wave_shape("auto", H, D, bs, T, phase)
+
+
 # (cache, H, D, bs, short, prompt): one case per launch shape, whole column widths and not; `short`: the first tokens only
 @pytest.mark.parametrize("cache,H,D,bs,short,prompt", [
     ("auto", 2, 64, 16, 500, 0), ("auto", 4, 128, 16, 0, 0), ("auto", 5, 104, 32, 0, 0), ("auto", 8, 128, 16, 0, 16), ("auto", 9, 72, 64, 0, 1000),
