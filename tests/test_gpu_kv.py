@@ -9,6 +9,7 @@ independent implementation.
 """
 import json
 import os
+import random
 
 import numpy as np
 import pytest
@@ -1108,15 +1109,16 @@ def test_paged_append_both_tile_widths(width, monkeypatch):
         hooks.emm_hook_set_move_variant(old)
 
 
-@pytest.mark.parametrize("cols,fused", [(1, 1), (1, 2), (2, 1), (2, 2), (3, 1), (3, 2)],
+@pytest.mark.parametrize("cols,fused", [(1, 1), (1, 2), (2, 1), (2, 2), (3, 1), (3, 2), (3, 5), (3, 6)],
                          ids=["128 row elements, K and V in one wave", "128 row elements, K and V in two waves",
                               "32 row elements, one wave", "32 row elements, two waves",
-                              "256 row elements, one wave", "256 row elements, two waves"])
-def test_paged_append_one_wave_kernel_every_wave_shape(cols, fused, monkeypatch):
-    """16-bit caches with aligned sources and a power-of-two block size from 16 on take the kernel of one-wave
-    workgroups, which picks how many row elements a wave takes, and whether K and V share a wave, by launch size;
-    here each shape is forced on launches of either size: rows that end inside a column, strided sources, prompts
-    on and off the token-tile grid, block size 32 and 64."""
+                              "256 row elements, one wave", "256 row elements, two waves",
+                              "64 row elements, one wave", "64 row elements, two waves"])
+def test_paged_append_forced_column_widths(cols, fused, monkeypatch):
+    """The column widths of the kernel of independent waves, K and V in one wave or in two, forced on launches of any
+    size in the form the hooks library can force: workgroups of one wave, rows requested when the slots are known, every
+    column guarded (the forms that a launch chooses by itself are run by the tests of its rules). Rows that end inside a
+    column, strided sources, prompts on and off the token-tile grid, block size 32 and 64."""
     hooks = _lib.load_hooks()
     monkeypatch.setattr(_lib, "_lib", hooks)
     old = hooks.emm_hook_set_move_variant((cols << 29) | (fused << 20))
@@ -1127,7 +1129,7 @@ def test_paged_append_one_wave_kernel_every_wave_shape(cols, fused, monkeypatch)
                 (torch.float16, 80, 16, 3, 40, 300, 4, 8), (torch.bfloat16, 48, 32, 2, 64, 700, 1, 8),
                 (torch.bfloat16, 60, 64, 1, 72, 900, 15, 0), (torch.bfloat16, 30, 16, 20, 128, 100, 1, 0),
                 (torch.float16, 40, 16, 1, 8, 333, 0, 0)]:
-            say(f"paged append, one-wave kernel, column code {cols}, fused code {fused}: {dtype} NB={NB} bs={bs} H={H} D={D} "
+            say(f"paged append, forced width, column code {cols}, fused code {fused}: {dtype} NB={NB} bs={bs} H={H} D={D} "
                 f"T={T} pad={pad}")
             g = torch.Generator().manual_seed(NB * 7 + T + cols)
             slots = paged_slots(NB, bs, T, seed=T + 1, phase=phase)
@@ -1431,6 +1433,66 @@ def test_paged_append_partial_runs_at_every_place(cache, H, D, bs, short, prompt
         else:
             orc.c_reshape_and_cache_paged(key, value, kc, vc, slots, float(ks), float(vs))
     assert same_bits(kc_g, kc) and same_bits(vc_g, vc)
+
+
+def _runs_beside_invalid_slots(NB, bs, T, seed):
+    """Runs of 6 to 16 tokens inside a window, each with entries that have to be skipped inside it, in front of it or behind
+    it: padding, slots past the pool, and slots past 2^32 whose low words would continue the run."""
+    r = random.Random(seed)
+    end, far, slots, k = NB * bs, 1 << 32, [], 0
+    blocks = list(range(NB - 1))
+    r.shuffle(blocks)
+    slots += range(end - 9, end + 3)  # nine slots, then three past the pool
+    while len(slots) < T:
+        n = 6 + r.randrange(11)
+        first = blocks.pop() * bs + 16 * r.randrange(bs // 16) + r.randrange(17 - n)
+        run = list(range(first, first + n))
+        i = r.randrange(n)
+        bad = (-1, end + r.randrange(1000), run[i] + far, -far + run[i])[k % 4]
+        kind = k % 7
+        if kind == 1: run[i] = bad
+        if kind == 2: run = [first - 1 + far] + run
+        if kind == 3: run = run + [first + n + far]
+        if kind == 4: run = [s + far for s in run]  # none of it
+        if kind == 5: run = [bad] + run + [bad]
+        if kind == 6: run = run[:i] + [bad] + run[i:]
+        slots += run
+        k += 1
+    return torch.tensor(slots[:T], dtype=torch.long)
+
+
+# (cache, H, D, bs, T, layers): the wave shapes that form partial runs, 16-bit 64 wide with K and V apart and in one wave, 256 and
+# 128 wide, fp8 64 wide with early and late rows, and the launches for all layers by either policy
+@pytest.mark.parametrize("cache,H,D,bs,T,layers", [
+    ("auto", 4, 128, 16, 1500, 1), ("auto", 4, 128, 16, 3200, 1), ("auto", 5, 104, 32, 2700, 1), ("auto", 8, 128, 16, 1700, 1), ("auto", 9, 120, 16, 1400, 1),
+    ("auto", 11, 120, 16, 4000, 1), ("auto", 16, 128, 32, 4000, 1), ("auto", 17, 120, 16, 3990, 1), ("fp8", 4, 128, 16, 2300, 1), ("fp8_sat", 5, 112, 64, 2000, 1),
+    ("fp8", 8, 128, 16, 3300, 1), ("auto", 4, 128, 16, 900, 3), ("auto", 4, 128, 16, 1900, 3), ("auto", 5, 104, 32, 1500, 3), ("fp8_sat", 4, 128, 16, 1200, 3)])
+def test_paged_append_runs_beside_slots_to_skip(cache, H, D, bs, T, layers):
+    say(f"paged append, runs beside slots to skip: {cache} H={H} D={D} bs={bs} T={T} layers={layers}")
+    NB = T // 6 + 40
+    slots = _runs_beside_invalid_slots(NB, bs, T, T + H)
+    inside = torch.where(slots < NB * bs, slots, -1)
+    assert (slots >= 1 << 32).sum() > T // 20 and (inside >= 0).sum() > T // 2
+    dtype = torch.bfloat16 if cache != "auto" or T % 200 else torch.float16
+    g = torch.Generator().manual_seed(T + H)
+    keys, values = ([(torch.randn((T, H, D), generator=g) * 30).to(dtype) for _ in range(layers)] for _ in range(2))
+    caches = [paged_caches_cpu(NB, H, D, bs, dtype if cache == "auto" else torch.uint8, fill_mod=31 + l) for l in range(layers)]
+    kcs, vcs = ([c[i].to(DEV) for c in caches] for i in range(2))
+    ks, vs = torch.linspace(0.03, 0.09, layers), torch.linspace(0.4, 0.2, layers)
+    if layers > 1:
+        cache_ops.paged_layered_append([k.to(DEV) for k in keys], [v.to(DEV) for v in values], kcs, vcs, cache, ks, vs)(slots.to(DEV))
+    else:
+        scales = () if cache == "auto" else (cache, ks.to(DEV), vs.to(DEV))
+        cache_ops.reshape_and_cache(keys[0].to(DEV), values[0].to(DEV), kcs[0], vcs[0], slots.to(DEV), *scales)
+    for l, (kc, vc) in enumerate(caches):
+        if cache == "auto":
+            orc.c_reshape_and_cache_paged(keys[l], values[l], kc, vc, inside)
+        elif cache == "fp8":
+            orc.c_reshape_and_cache_paged(keys[l], values[l], kc, vc, inside, float(ks[l]), float(vs[l]))
+        else:  # the bytes of the saturating cast, placed by the byte-copying reference
+            k8, v8 = (torch.from_numpy(orc.c_quant_fp8_sat(x, float(sc[l])).reshape(T, H, D).copy()) for x, sc in ((keys[l], ks), (values[l], vs)))
+            orc.ref_reshape_and_cache_paged(k8, v8, kc, vc, inside)
+        assert same_bits(kcs[l], kc) and same_bits(vcs[l], vc), f"layer {l}"
 
 
 @pytest.mark.parametrize("bs,seqs,chunk,pad", [(16, 1, 0, 0), (16, 24, 0, 3), (16, 239, 0, 0), (16, 240, 0, 0), (12, 400, 1000, 7),
