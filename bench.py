@@ -11,7 +11,8 @@ unpack every buffer into a second, independently allocated pool under a differen
 table (``KVWorker.write_kv_blocks``, one call per request). Everything is resident in
 HBM before the timed region (pools, block tables); values are synthetic N(0, 0.5).
 
-Prints ONE JSON line. ``value`` is whole-job GB/s = algorithmic bytes (read + write of
+Prints ONE JSON line on stdout. Of ``extra`` below it holds the rates only (``extra_GBps``); the whole record goes to
+``--details FILE`` or, without it, to stderr. ``value`` is whole-job GB/s = algorithmic bytes (read + write of
 pack and of unpack = 4 x payload) / wall time of the timed steps. ``roofline`` prices the
 block-move kernel (pack and unpack are two instances of the same kernel) against the
 8 TB/s HBM peak from HIP-event times of its launches inside the timed region.
@@ -77,6 +78,7 @@ def parse():
     ap.add_argument("--no-append-context", action="store_true",
                     help="skip extra.append.in_context (HIP graphs that fork over several streams or contain library GEMMs; "
                          "rocprofv3 --pmc has crashed replaying them)")
+    ap.add_argument("--details", default="", help="file for the whole record (default: a JSON line on stderr)")
     ap.add_argument("--calibrate-copy", action="store_true",
                     help="also launch one plain 1 GiB copy with the same tile engine (a kernel of known traffic, "
                          "for scaling rocprofv3 FETCH_SIZE / WRITE_SIZE readings)")
@@ -552,7 +554,27 @@ def main():
         result["cpu_baseline"] = cpu_baseline(tables, L, bs, H, D, dtype)
         result["cpu_baseline"]["append"] = cpu_baseline_append()
         result["cpu_baseline"]["cfg1"] = cpu_baseline_cfg1()
-    print(json.dumps(result), flush=True)
+    # The record of all sections is some 25 KB: it goes to a file or to stderr, and the one line on stdout keeps the headline and of
+    # the sections their rates.
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(result, f, indent=1)
+    else:
+        print(json.dumps(result), file=sys.stderr, flush=True)
+    line = {k: v for k, v in result.items() if k != "extra"}
+    line["extra_GBps"] = rates(extra)
+    print(json.dumps(line), flush=True)
+
+
+def rates(record):
+    """The GB/s of every measurement in a nested record, whole numbers, under the same names."""
+    if not isinstance(record, dict):
+        return None
+    for key in ("GBps", "value_GBps"):
+        if key in record:
+            return round(record[key])
+    inner = {k: rates(v) for k, v in record.items()}
+    return {k: v for k, v in inner.items() if v is not None} or None
 
 
 # ---------------------------------------------------------------------------------------------- secondary shapes
@@ -941,15 +963,17 @@ def append_bench(kv, NB, bs, H, D, k_scales, v_scales, dev, T=8448):
     step_bytes = L * (valid * 2 * row * (2 + kv[0].element_size()) + 8 * T)
     ks = [None] * L if not fp8 else [k_scales[l:l + 1] for l in range(L)]
     vs = [None] * L if not fp8 else [v_scales[l:l + 1] for l in range(L)]
-    kernel = "emm_append_fp8_kernel" if fp8 else "emm_append_kernel"  # one launch for all layers
-    per_layer_kernel = kernel if fp8 else "emm_append_tile_kernel"
+    # what T = 8448 rows (per layer and in one launch) and 256 rows take
+    kernel = "emm_append_fp8_kernel" if fp8 else "emm_append_kernel"
+    whole_kernel = "emm_append_fp8_half_kernel" if fp8 else "emm_append_kernel"
+    per_layer_kernel = "emm_append_fp8_kernel" if fp8 else "emm_append_tile_kernel"
 
     def per_layer():
         for l in range(L):
             cache_ops.reshape_and_cache_flash(keys[l], values[l], kv[l][0], kv[l][1], slots, mode, ks[l], vs[l])
 
     def entry(ms, launches):
-        return rec(step_bytes, ms, launches, kernel if launches == 1 else per_layer_kernel, tokens_per_s=round(valid / (ms * 1e-3)))
+        return rec(step_bytes, ms, launches, whole_kernel if launches == 1 else per_layer_kernel, tokens_per_s=round(valid / (ms * 1e-3)))
 
     def graphed(fn):
         graph = torch.cuda.CUDAGraph()
