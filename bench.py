@@ -966,7 +966,7 @@ def append_bench(kv, NB, bs, H, D, k_scales, v_scales, dev, T=8448):
     # what T = 8448 rows (per layer and in one launch) and 256 rows take
     kernel = "emm_append_fp8_kernel" if fp8 else "emm_append_kernel"
     whole_kernel = "emm_append_fp8_half_kernel" if fp8 else "emm_append_kernel"
-    per_layer_kernel = "emm_append_fp8_kernel" if fp8 else "emm_append_tile_kernel"
+    per_layer_kernel = "emm_append_fp8_kernel" if fp8 else "emm_append_kernel"
 
     def per_layer():
         for l in range(L):
