@@ -1466,7 +1466,8 @@ def _runs_beside_invalid_slots(NB, bs, T, seed):
 @pytest.mark.parametrize("cache,H,D,bs,T,layers", [
     ("auto", 4, 128, 16, 1500, 1), ("auto", 4, 128, 16, 3200, 1), ("auto", 5, 104, 32, 2700, 1), ("auto", 8, 128, 16, 1700, 1), ("auto", 9, 120, 16, 1400, 1),
     ("auto", 11, 120, 16, 4000, 1), ("auto", 16, 128, 32, 4000, 1), ("auto", 17, 120, 16, 3990, 1), ("fp8", 4, 128, 16, 2300, 1), ("fp8_sat", 5, 112, 64, 2000, 1),
-    ("fp8", 8, 128, 16, 3300, 1), ("auto", 4, 128, 16, 900, 3), ("auto", 4, 128, 16, 1900, 3), ("auto", 5, 104, 32, 1500, 3), ("fp8_sat", 4, 128, 16, 1200, 3)])
+    ("fp8", 8, 128, 16, 3300, 1), ("auto", 4, 128, 16, 900, 3), ("auto", 4, 128, 16, 1900, 3), ("auto", 5, 104, 32, 1500, 3), ("fp8_sat", 4, 128, 16, 1200, 3),
+    ("fp8", 32, 128, 16, 1488, 2), ("fp8_sat", 32, 128, 32, 1505, 2)])
 def test_paged_append_runs_beside_slots_to_skip(cache, H, D, bs, T, layers):
     say(f"paged append, runs beside slots to skip: {cache} H={H} D={D} bs={bs} T={T} layers={layers}")
     NB = T // 6 + 40
