@@ -1313,7 +1313,8 @@ def test_paged_append_on_both_sides_of_its_rules(cache, H, D, bs, T, phase):
     test_paged_append_every_dispatched_wave_shape(cache, H, D, bs, T, phase)
 
 
-# all layers in one launch: pieces = ceil(T / 16) * ceil(H * D / 128), few and many; rows that 64-element waves cut evenly and not
+# all layers in one launch: pieces = ceil(T / 16) * ceil(H * D / 128), both sides of 448 (16-bit), few and many; rows that 64-element
+# waves cut evenly and not
 @pytest.mark.parametrize("cache,H,D,bs,T,phase", [
     ("auto", 5, 104, 16, 1424, 3), ("auto", 5, 104, 16, 1425, 0), ("auto", 5, 104, 32, 3680, 1), ("auto", 9, 120, 16, 784, 2),
     ("auto", 9, 120, 64, 785, 5), ("auto", 2, 40, 16, 33, 6),
@@ -1377,8 +1378,8 @@ def test_paged_append_of_many_short_prompts(layers, H, D, bs, q, step):
         assert same_bits(kcs[l], kc) and same_bits(vcs[l], vc), f"layer {l}"
 
 
-# the wave shapes change past 32 pieces, at 320 and 768 (16-bit), at 2600 with rows of up to 512, up to 1024 and more elements,
-# at 512 and 1600 (fp8)
+# the wave shapes change past 32 pieces, at 320 and 768 (16-bit), at 2600 with rows of up to 512, up to 1024 and more elements (those
+# again at 4000: below), at 512 and 1600 (fp8)
 @pytest.mark.parametrize("cache,H,D,bs,T,phase", [
     ("auto", 4, 128, 16, 128, 3), ("auto", 4, 128, 16, 129, 5), ("auto", 5, 104, 16, 1008, 2), ("auto", 5, 104, 16, 1009, 0), ("auto", 4, 128, 32, 3056, 9),
     ("auto", 4, 128, 16, 3057, 1), ("auto", 9, 120, 16, 1360, 0), ("auto", 9, 120, 16, 1361, 4), ("auto", 13, 128, 16, 3184, 7), ("auto", 13, 128, 16, 3185, 7),
